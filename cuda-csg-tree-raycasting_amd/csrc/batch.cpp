@@ -35,6 +35,7 @@ struct Chunk {
   uint2* heavy = nullptr;
   csgray::RenderParams params{};
   csgray::LaunchShape shape{};
+  const void* fn = nullptr;  // the captured render kernel
   hipGraphNode_t node = nullptr;
   hipGraphNode_t coopNode = nullptr;
 };
@@ -186,12 +187,13 @@ csg_status Stage(csg_batch* b) {
     if (cnt > ch.cap) return Fail(CSG_E_ARG, "csg_batch: chunk capacity exceeded");
     int64_t base = 0;
     int32_t depth = 1, maxOps = 1, maxLeaves = 1;
-    bool anyInBoxes = false;
+    bool anyInBoxes = false, anyGroups = false;
     for (int32_t i = 0; i < cnt; i++) {
       const csg_job& j = b->jobs[plan.order[start + i]];
       maxOps = std::max(maxOps, j.scene->dev.nOps);
       maxLeaves = std::max(maxLeaves, j.scene->dev.opLeaves);
       anyInBoxes |= j.scene->dev.conservative != 0;
+      anyGroups |= HasTileGroups(j.scene);
       const csg_status st = BuildJob(j.scene, &j.camera, &j.light, &j.phong, j.width, j.height, &j.out, &b->opts,
                                      b->device, base, &ch.hostJobs[i]);
       if (st != CSG_OK) return st;
@@ -211,7 +213,7 @@ csg_status Stage(csg_batch* b) {
     if (e != hipSuccess) return FailHip(e, "choosing the launch shape");
     csgray::FitGridToTiles(&ch.shape, base);
     p.totalWaves = static_cast<uint32_t>(ch.shape.grid) * static_cast<uint32_t>(ch.shape.block / 64);
-    PrepareCoop(b->cfg, maxOps, maxLeaves, anyInBoxes, ch.heavy, ch.shape, &p);
+    PrepareCoop(b->cfg, maxOps, maxLeaves, anyInBoxes, anyGroups, ch.heavy, ch.shape, &p);
   }
   return CSG_OK;
 }
@@ -271,17 +273,34 @@ csg_status Capture(csg_batch* b) {
   for (Chunk& ch : b->chunks) {
     ch.node = nullptr;
     ch.coopNode = nullptr;
+    ch.fn = csgray::MainLaunch(ch.params, b->cfg, ch.shape).fn;
   }
-  for (hipGraphNode_t nd : nodes) {
+  // A kernel node's launch parameters (null for another kind of node).
+  auto paramsOf = [](hipGraphNode_t nd) -> const csgray::RenderParams* {
     hipGraphNodeType type;
-    if (hipGraphNodeGetType(nd, &type) != hipSuccess || type != hipGraphNodeTypeKernel) continue;
+    if (hipGraphNodeGetType(nd, &type) != hipSuccess || type != hipGraphNodeTypeKernel) return nullptr;
     hipKernelNodeParams kp{};
-    if (hipGraphKernelNodeGetParams(nd, &kp) != hipSuccess || !kp.kernelParams) continue;
-    const auto* p = static_cast<const csgray::RenderParams*>(kp.kernelParams[0]);
+    if (hipGraphKernelNodeGetParams(nd, &kp) != hipSuccess || !kp.kernelParams) return nullptr;
+    return static_cast<const csgray::RenderParams*>(kp.kernelParams[0]);
+  };
+  for (hipGraphNode_t nd : nodes) {
+    const csgray::RenderParams* p = paramsOf(nd);
+    if (!p) continue;
+    // a chunk's cooperative kernel follows its render kernel directly
+    bool follows = false;
+    size_t deps = 0;
+    if (hipGraphNodeGetDependencies(nd, nullptr, &deps) == hipSuccess && deps > 0) {
+      std::vector<hipGraphNode_t> before(deps);
+      e = hipGraphNodeGetDependencies(nd, before.data(), &deps);
+      if (e != hipSuccess) return FailHip(e, "hipGraphNodeGetDependencies");
+      for (hipGraphNode_t b4 : before) {
+        const csgray::RenderParams* bp = paramsOf(b4);
+        follows |= bp && bp->queue == p->queue;
+      }
+    }
     for (Chunk& ch : b->chunks) {
       if (p->queue != ch.queue) continue;
-      // the render kernel runs on the chunk's launch shape, the cooperative one on 64-lane groups
-      if (kp.blockDim.x == 64 && ch.shape.block != 64) ch.coopNode = nd;
+      if (follows) ch.coopNode = nd;
       else ch.node = nd;
     }
   }
@@ -294,39 +313,34 @@ csg_status Capture(csg_batch* b) {
 
 // Points each kernel node of the instantiated graph at its chunk's current
 // launch parameters.  The graph is captured again instead when the nodes no
-// longer match the chunks (another chunk count, deferral switched on or off)
+// longer match the chunks (another chunk count, deferral switched on or off,
+// another render kernel)
 // or a kernel needs more than 64 KB of LDS, whose launch attribute only a
 // direct launch sets.
 csg_status PatchNodes(csg_batch* b) {
   for (const Chunk& ch : b->chunks) {
-    const size_t coopLds = csgray::CoopLaunchLds(ch.params);
-    if (!ch.node || (ch.params.budget > 0) != (ch.coopNode != nullptr) || ch.shape.lds > 64 * 1024 ||
-        (ch.params.budget > 0 && coopLds > 64 * 1024))
+    const csgray::KernelLaunch coop = csgray::CoopLaunch(ch.params, b->cfg);
+    const csgray::KernelLaunch main = csgray::MainLaunch(ch.params, b->cfg, ch.shape);
+    if (!ch.node || (coop.fn != nullptr) != (ch.coopNode != nullptr) || main.fn != ch.fn ||
+        main.lds > 64 * 1024 || coop.lds > 64 * 1024)
       return Capture(b);
   }
   for (Chunk& ch : b->chunks) {
-    hipKernelNodeParams kp{};
-    hipError_t e = hipGraphKernelNodeGetParams(ch.node, &kp);
-    if (e != hipSuccess) return FailHip(e, "hipGraphKernelNodeGetParams");
-    void* args[1] = {&ch.params};
-    kp.kernelParams = args;
-    kp.extra = nullptr;
-    kp.gridDim = dim3(ch.shape.grid);
-    kp.blockDim = dim3(ch.shape.block);
-    kp.sharedMemBytes = static_cast<unsigned int>(ch.shape.lds);
-    e = hipGraphExecKernelNodeSetParams(b->exec, ch.node, &kp);
-    if (e != hipSuccess) return FailHip(e, "hipGraphExecKernelNodeSetParams");
-    if (ch.coopNode) {
-      hipKernelNodeParams cp{};
-      e = hipGraphKernelNodeGetParams(ch.coopNode, &cp);
+    const std::pair<hipGraphNode_t, csgray::KernelLaunch> parts[2] = {
+        {ch.node, csgray::MainLaunch(ch.params, b->cfg, ch.shape)},
+        {ch.coopNode, csgray::CoopLaunch(ch.params, b->cfg)}};
+    for (const auto& [node, launch] : parts) {
+      if (!node) continue;
+      hipKernelNodeParams kp{};
+      hipError_t e = hipGraphKernelNodeGetParams(node, &kp);
       if (e != hipSuccess) return FailHip(e, "hipGraphKernelNodeGetParams");
-      void* cargs[1] = {&ch.params};
-      cp.kernelParams = cargs;
-      cp.extra = nullptr;
-      cp.gridDim = dim3(ch.params.coopWaves);
-      cp.blockDim = dim3(64);
-      cp.sharedMemBytes = static_cast<unsigned int>(csgray::CoopLaunchLds(ch.params));
-      e = hipGraphExecKernelNodeSetParams(b->exec, ch.coopNode, &cp);
+      void* args[1] = {&ch.params};
+      kp.kernelParams = args;
+      kp.extra = nullptr;
+      kp.gridDim = dim3(launch.grid);
+      kp.blockDim = dim3(launch.block);
+      kp.sharedMemBytes = static_cast<unsigned int>(launch.lds);
+      e = hipGraphExecKernelNodeSetParams(b->exec, node, &kp);
       if (e != hipSuccess) return FailHip(e, "hipGraphExecKernelNodeSetParams");
     }
   }
@@ -421,8 +435,10 @@ csg_status csg_batch_autotune(csg_batch* b, int32_t reps, void* stream, csg_batc
   csg_status st = CSG_OK;
   std::vector<int32_t> splits{0};
   if (const int32_t half = HalfWorkDepth(b)) splits.push_back(half);
+  // block 0: the launch a batch starts with, which classifies whole tiles
+  // where the options allow it
   for (int32_t split : splits)
-  for (int32_t block : {256, 512, 1024}) {
+  for (int32_t block : {0, 256, 512, 1024}) {
     for (int32_t walk : {0, 1}) {
       for (bool heavy : {false, true}) {
         csg_render_opts o = base;
@@ -435,6 +451,9 @@ csg_status csg_batch_autotune(csg_batch* b, int32_t reps, void* stream, csg_batc
         if (st == CSG_OK) st = WaitStaged(b);
         if (st == CSG_OK) st = EnsureChunks(b);
         if (st == CSG_OK) st = Stage(b);
+        if (st == CSG_OK && block == 0 &&
+            std::none_of(b->chunks.begin(), b->chunks.end(), [](const Chunk& c) { return c.params.tileSlots > 0; }))
+          continue;
         if (st == CSG_OK) st = Upload(b, hs);
         if (st == CSG_OK) st = LaunchDirect(b, hs);  // warm-up
         if (st != CSG_OK) break;
@@ -476,7 +495,7 @@ csg_status csg_batch_autotune(csg_batch* b, int32_t reps, void* stream, csg_batc
   if (st != CSG_OK) return st;
   if (st2 != CSG_OK) return st2;
   if (chosen) {
-    chosen->block = b->opts.block;
+    chosen->block = b->opts.block != 0 ? b->opts.block : b->chunks[0].shape.block;
     chosen->tile_walk = b->opts.tile_walk;
     chosen->heaviest_first = b->heaviestFirst ? 1 : 0;
     chosen->ms = best;

@@ -40,9 +40,10 @@ size_t Align256(size_t n) { return (n + 255) & ~static_cast<size_t>(255); }
 // One device allocation holding the scene arrays back to back.
 csg_status Upload(csg_scene* s) {
   const csgray::FlatScene& f = s->flat;
-  const std::vector<csgray::F4>* src[6] = {&f.ops, &f.primA, &f.primB, &f.primC, &f.ivOps, &f.walkOps};
-  size_t off[6], total = 0;
-  for (int k = 0; k < 6; k++) {
+  const std::vector<csgray::F4>* src[7] = {&f.ops,   &f.primA,   &f.primB,  &f.primC,
+                                             &f.ivOps, &f.walkOps, &f.tileOps};
+  size_t off[7], total = 0;
+  for (int k = 0; k < 7; k++) {
     off[k] = total;
     total += Align256(sizeof(csgray::F4) * src[k]->size());
   }
@@ -55,7 +56,7 @@ csg_status Upload(csg_scene* s) {
     return e == hipErrorOutOfMemory ? Fail(CSG_E_OOM, "hipMalloc of the scene failed") : FailHip(e, "hipMalloc");
   }
   char* base = static_cast<char*>(s->dmem);
-  for (int k = 0; k < 6; k++) {
+  for (int k = 0; k < 7; k++) {
     if (src[k]->empty()) continue;
     e = hipMemcpy(base + off[k], src[k]->data(), sizeof(csgray::F4) * src[k]->size(), hipMemcpyHostToDevice);
     if (e != hipSuccess) return FailHip(e, "hipMemcpy of the scene");
@@ -66,6 +67,7 @@ csg_status Upload(csg_scene* s) {
   s->dev.primC = reinterpret_cast<const float4*>(base + off[3]);
   s->dev.ivOps = f.ivOps.empty() ? nullptr : reinterpret_cast<const float4*>(base + off[4]);
   s->dev.walkOps = f.walkOps.empty() ? nullptr : reinterpret_cast<const float4*>(base + off[5]);
+  s->dev.tileOps = f.tileOps.empty() ? s->dev.ivOps : reinterpret_cast<const float4*>(base + off[6]);
   s->dev.rootDesc = f.rootDesc;
   s->dev.nOps = f.nOps;
   s->dev.nPrims = f.nPrims;
@@ -188,9 +190,10 @@ int32_t DefaultCoopGraceMille(int64_t waves, int64_t tiles, bool batched, bool l
   return static_cast<int32_t>(std::min<int64_t>(std::max<int64_t>(g, 5), batched ? 1000000 : 3000));
 }
 
-void PrepareCoop(const LaunchConfig& cfg, int32_t maxOps, int32_t maxLeaves, bool anyInBoxes, uint2* heavy,
-                 const LaunchShape& shape, RenderParams* p) {
+void PrepareCoop(const LaunchConfig& cfg, int32_t maxOps, int32_t maxLeaves, bool anyInBoxes, bool anyGroups,
+                 uint2* heavy, const LaunchShape& shape, RenderParams* p) {
   p->budget = 0;
+  PlanTiles(cfg, anyGroups, p);
   if (!heavy) return;
   const bool lists = CoopLists(cfg, anyInBoxes);
   const CoopPlan c = PlanCoop(cfg, maxOps, maxLeaves, lists);
@@ -411,6 +414,7 @@ void csg_phong_default(csg_phong* ph) {  // RaycastingKernels.cu:71-74, 109
 namespace csgray {
 namespace rt {
 csg_status ParseOpts(const csg_render_opts* opts, csgray::LaunchConfig* cfg) {
+  cfg->tiles = true;
   if (!opts) return CSG_OK;
   if (opts->mode != CSG_MODE_EXACT && opts->mode != CSG_MODE_FAST) return Fail(CSG_E_ARG, "csg_render: unknown mode");
   cfg->mode = opts->mode == CSG_MODE_EXACT ? csgray::Mode::kExact : csgray::Mode::kFast;
@@ -433,6 +437,10 @@ csg_status ParseOpts(const csg_render_opts* opts, csgray::LaunchConfig* cfg) {
   if (opts->coop_grace > 100000) return Fail(CSG_E_ARG, "coop_grace above 100000 percent");
   cfg->coopGrace = opts->coop_grace;
   cfg->coopIntervals = opts->coop_intervals >= 0;
+  // Whole tiles are classified unless the caller shapes the per-lane launch
+  // (the hand-over, the workgroup, the reference's boxes).
+  cfg->tiles = opts->coop_budget == 0 && opts->coop_when == 0 && opts->coop_grace == 0 && cfg->coopIntervals &&
+               opts->tight_boxes >= 0 && opts->block == 0;
   return CSG_OK;
 }
 
@@ -691,7 +699,8 @@ csg_status csg_render_ex(const csg_scene* s, const csg_camera* cam, const csg_li
     const csg_status hsd = HeavyFor(dev, hs, &heavy);
     if (hsd != CSG_OK) return hsd;
   }
-  PrepareCoop(cfg, s->dev.nOps, s->dev.opLeaves, s->dev.conservative != 0, heavy, shape, &p);
+  cfg.tiles = cfg.tiles && cfg.sceneInLds == -1 && !p.tileOrder && TilesPay(s, p.numTiles);
+  PrepareCoop(cfg, s->dev.nOps, s->dev.opLeaves, s->dev.conservative != 0, HasTileGroups(s), heavy, shape, &p);
   e = csgray::LaunchRender(p, cfg, shape, hs);
   if (e != hipSuccess) return FailHip(e, "render launch");
   return CSG_OK;
@@ -761,13 +770,14 @@ csg_status csg_render_batch(const csg_job* jobs, int32_t njobs, const csg_render
       if (hsd != CSG_OK) return hsd;
     }
     int32_t maxOps = 1, maxLeaves = 1;
-    bool anyInBoxes = false;
+    bool anyInBoxes = false, anyGroups = false;
     for (int32_t i = 0; i < n; i++) {
       maxOps = std::max(maxOps, jobs[start + i].scene->dev.nOps);
       maxLeaves = std::max(maxLeaves, jobs[start + i].scene->dev.opLeaves);
       anyInBoxes |= jobs[start + i].scene->dev.conservative != 0;
+      anyGroups |= HasTileGroups(jobs[start + i].scene);
     }
-    PrepareCoop(cfg, maxOps, maxLeaves, anyInBoxes, heavy, shape, &p);
+    PrepareCoop(cfg, maxOps, maxLeaves, anyInBoxes, anyGroups, heavy, shape, &p);
     e = csgray::LaunchRender(p, cfg, shape, hs);
     if (e != hipSuccess) return FailHip(e, "batched render launch");
   }

@@ -22,6 +22,7 @@ struct DevScene {
   uint32_t conservative;  // 1: every primitive lies inside its box (interval classification applies)
   const float4* ivOps;    // operator records with fast mode's culling boxes (tight where the reference allows)
   const float4* walkOps;  // interval classification's records: ivOps with Union groups flattened (scene.hpp)
+  const float4* tileOps;  // the tile kernel's: ivOps with the large groups of walkOps
 };
 
 // One render job: a scene seen by one camera at one resolution, with its
@@ -80,6 +81,8 @@ struct RenderParams {
   uint32_t* resume;
   uint32_t resumeBytes;
   int32_t cacheOps;           // plain global-memory launches: operator records [0, cacheOps) staged in LDS
+  int32_t tileSlots;          // the tile kernel's list slots a lane (0: not used)
+  int32_t tileGroups;         // some scene has Union groups in its tileOps
 };
 // queue words: [1] render workgroups done, [2] heavy rays, [4] coop waves done, [6..7] heavy rays handed
 // over on this stream so far (64-bit), [8..9] of those, the ones finished from boundary lists; on their own cache line, [32..33] time the first tile was taken,
@@ -118,6 +121,7 @@ struct LaunchConfig {
   bool coopEager = false;   // hand rays over as soon as the budget is spent, not only after the queue drains
   int32_t coopGrace = 0;    // 0: default; < 0: none; else percent (see RenderParams::coopGrace)
   bool coopIntervals = true;  // interval classification of heavy rays where it applies
+  bool tiles = false;         // classify whole tiles (PlanTiles) where the mode allows
 };
 
 // Launch geometry chosen for a scene: workgroup size, grid, LDS bytes.
@@ -147,6 +151,31 @@ hipError_t ChooseShape(int32_t depth, size_t sceneBytes, const LaunchConfig& cfg
 
 // Compute units, LDS bytes per workgroup and per CU of the current device.
 hipError_t DeviceShapeLimits(int* computeUnits, size_t* ldsPerBlock, size_t* ldsPerCu = nullptr);
+
+// Tile kernel (tile.hpp): entries of a lane's list stack and waves a CU holds,
+// with Union groups and without, and one wave's LDS for trees of `depth`
+// operator levels.
+constexpr int32_t kTileSlots = 26, kTilePlainSlots = 16;
+constexpr int32_t kMaxTileGrid = 0x3FFFFFF;  // a grid has fewer than 2^32 threads
+constexpr size_t TileLds(int32_t slots, int32_t depth) {
+  const size_t bytes = 512 * static_cast<size_t>(slots + 2) + 64 + 144 + 64 * static_cast<size_t>(depth > 0 ? depth : 1);
+  return (bytes + 15) & ~static_cast<size_t>(15);
+}
+
+// Fills the tile kernel's fields of `p` (numTiles and stackSlots set):
+// tileSlots stays 0 where it does not apply.  `groups`: some scene of the
+// launch has Union groups in its tileOps.
+void PlanTiles(const LaunchConfig& cfg, bool groups, RenderParams* p);
+
+// One kernel of a launch: the kernel that renders the frame, and the
+// cooperative one (fn null when none follows).
+struct KernelLaunch {
+  const void* fn = nullptr;
+  uint32_t grid = 0, block = 0;
+  size_t lds = 0;
+};
+KernelLaunch MainLaunch(const RenderParams& p, const LaunchConfig& cfg, const LaunchShape& s);
+KernelLaunch CoopLaunch(const RenderParams& p, const LaunchConfig& cfg);
 
 // Enqueues one launch on `stream` with the given shape (p.numJobs == 0:
 // plain render of p.job; otherwise the batch in p.jobs).

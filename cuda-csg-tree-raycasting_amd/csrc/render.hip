@@ -262,6 +262,25 @@ __device__ __forceinline__ bool SphereRoots(const RayF& r, const float4& a, floa
   return true;
 }
 
+// The same without a branch (the roots of a ray that misses are NaN).
+template <bool kFast>
+__device__ __forceinline__ bool RootsOfSphere(const RayF& r, const float4& a, float& t0, float& t1) {
+  const float ocx = r.ox - a.x, ocy = r.oy - a.y, ocz = r.oz - a.z;
+  const float b = ocx * r.dx + ocy * r.dy + ocz * r.dz;
+  float disc;
+  if (kFast) {
+    const float fx = fmaf(-b, r.dx, ocx), fy = fmaf(-b, r.dy, ocy), fz = fmaf(-b, r.dz, ocz);
+    disc = a.w * a.w - (fx * fx + fy * fy + fz * fz);
+  } else {
+    const float c = (ocx * ocx + ocy * ocy + ocz * ocz) - a.w * a.w;
+    disc = b * b - c;
+  }
+  const float sq = kFast ? __builtin_amdgcn_sqrtf(disc) : sqrtf(disc);
+  t0 = (-b - sq);
+  t1 = (-b + sq);
+  return !(disc < 0);
+}
+
 // The sphere's hit record at root `temp` (Enter where the outward normal
 // faces the ray).
 __device__ __forceinline__ Hit SphereAt(const RayF& r, const float4& a, uint32_t prim, float temp) {
@@ -302,6 +321,106 @@ __device__ __forceinline__ Hit SphereHit(const RayF& r, const float4& a, uint32_
 // keeps them near 1e-6.  Where the reference's clamp A = 1e-5 applies (rays
 // within 0.18 degrees of the axis) the clamped quadratic is kept:
 // (b^2 - A c) / A = -b tc - c.
+// A ray's two candidate crossings of a cylinder, in the order of the roots:
+// the side's root or, where that lies beyond a cap's plane, the cap (cap 1
+// bottom, 2 top); `skip` where the cap's plane is parallel to the ray.
+struct CylinderRoots {
+  float t[2], m[2];
+  uint32_t cap[2];
+  bool skip[2];
+  float Cx, Cy, Cz, vx, vy, vz;
+};
+
+// False when the ray misses the cylinder's side or passes both caps outside
+// (without a branch).
+template <bool kFast>
+__device__ __forceinline__ bool RootsOfCylinder(const RayF& r, const float4& a, const float4& bx, CylinderRoots& o) {
+  const float vx = bx.x, vy = bx.y, vz = bx.z, height = bx.w, radius = a.w;
+  const float hh = height / 2;
+  const float Cx = a.x - hh * vx, Cy = a.y - hh * vy, Cz = a.z - hh * vz;
+  const float OCx = r.ox - Cx, OCy = r.oy - Cy, OCz = r.oz - Cz;
+  const float dV = r.dx * vx + r.dy * vy + r.dz * vz;  // dot(d, V)
+  const float ocV = OCx * vx + OCy * vy + OCz * vz;  // dot(OC, V)
+  float t1, t2;
+  bool miss;
+  if (kFast) {
+    const float ex = r.dy * vz - r.dz * vy, ey = r.dz * vx - r.dx * vz, ez = r.dx * vy - r.dy * vx;
+    const float gx = OCy * vz - OCz * vy, gy = OCz * vx - OCx * vz, gz = OCx * vy - OCy * vx;
+    const float A0 = ex * ex + ey * ey + ez * ez;
+    const float A = fmaxf(A0, 0.00001f);
+    const float b = ex * gx + ey * gy + ez * gz;
+    const float tc = -b / A;
+    const float fx = fmaf(tc, ex, gx), fy = fmaf(tc, ey, gy), fz = fmaf(tc, ez, gz);
+    const float rr = radius * radius;
+    const float dp = A0 >= 0.00001f ? rr - (fx * fx + fy * fy + fz * fz)
+                                    : fmaf(-b, tc, rr - (gx * gx + gy * gy + gz * gz));
+    miss = dp < 0;
+    const float s = __builtin_amdgcn_sqrtf(dp * __builtin_amdgcn_rcpf(A));
+    t1 = tc - s;
+    t2 = tc + s;
+  } else {
+    const float A = fmaxf(1 - dV * dV, 0.00001f);
+    const float c = (OCx * OCx + OCy * OCy + OCz * OCz) - ocV * ocV - radius * radius;
+    const float dOC = r.dx * OCx + r.dy * OCy + r.dz * OCz;
+    const float b = (dOC - dV * ocV);
+    const float disc = b * b - A * c;
+    miss = disc < 0;
+    const float sq = sqrtf(disc);
+    t1 = (-b - sq) / (A);
+    t2 = (-b + sq) / (A);
+  }
+  const float m1 = t1 * dV + ocV;
+  const float m2 = t2 * dV + ocV;
+  miss |= ((m1 < 0) & (m2 < 0)) | ((m1 > height) & (m2 > height));
+
+  // dot(d, -V), dot(-OC, -V) and dot(-OCmMax, V) written out as the
+  // reference evaluates them.
+  const float dnV = r.dx * (-vx) + r.dy * (-vy) + r.dz * (-vz);
+  const float capBot = (-OCx) * (-vx) + (-OCy) * (-vy) + (-OCz) * (-vz);
+  const float Mx = (r.ox - a.x) - hh * vx, My = (r.oy - a.y) - hh * vy, Mz = (r.oz - a.z) - hh * vz;
+  const float capTop = (-Mx) * vx + (-My) * vy + (-Mz) * vz;
+  const float tBot = capBot / dnV, tTop = capTop / dV;
+  const bool flatBot = fabsf(dnV) < 0.0001f, flatTop = fabsf(dV) < 0.0001f;
+#pragma unroll
+  for (int k = 0; k < 2; k++) {
+    float t = k == 0 ? t1 : t2;
+    const float m = k == 0 ? m1 : m2;
+    const bool below = m < 0, above = m > height;
+    t = below & !flatBot ? tBot : t;
+    t = above & !flatTop ? tTop : t;
+    const uint32_t cap = above & !flatTop ? 2u : (below & !flatBot ? 1u : 0u);
+    const bool skip = (below & flatBot) | (above & flatTop);
+    o.t[k] = t;
+    o.m[k] = m;
+    o.cap[k] = cap;
+    o.skip[k] = skip;
+  }
+  o.Cx = Cx;
+  o.Cy = Cy;
+  o.Cz = Cz;
+  o.vx = vx;
+  o.vy = vy;
+  o.vz = vz;
+  return !miss;
+}
+
+// The cylinder's hit record at its k-th candidate.
+__device__ __forceinline__ Hit CylinderAt(const RayF& r, const CylinderRoots& o, uint32_t prim, int k) {
+  const float temp = o.t[k], m = o.m[k];
+  const uint32_t cap = o.cap[k];
+  float nx = ((r.ox + temp * r.dx) - o.Cx) - m * o.vx;
+  float ny = ((r.oy + temp * r.dy) - o.Cy) - m * o.vy;
+  float nz = ((r.oz + temp * r.dz) - o.Cz) - m * o.vz;
+  if (cap != 0) {
+    nx = cap == 1 ? -o.vx : o.vx;
+    ny = cap == 1 ? -o.vy : o.vy;
+    nz = cap == 1 ? -o.vz : o.vz;
+  }
+  const float dn = nx * r.dx + ny * r.dy + nz * r.dz;
+  const uint32_t f = (dn <= 0 ? kEnter : kExit) | (cap == 1 ? kFlag1 : (cap == 2 ? kFlag2 : 0u));
+  return Hit{temp, HitBits(f, kCylinderT, prim)};
+}
+
 template <bool kFast>
 __device__ __forceinline__ Hit CylinderHit(const RayF& r, const float4& a, const float4& bx, uint32_t prim,
                                            float tmin, Hit h) {
@@ -2118,6 +2237,8 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) Co
   }
 }
 
+#include "tile.hpp"
+
 constexpr int kMaxDepth = 64;
 
 constexpr size_t kStaticLds = 256;  // the action table and alignment slack
@@ -2141,24 +2262,25 @@ hipError_t AllowLds(const void* fn, size_t lds) {
 }
 
 template <bool kFast, bool kCount, bool kLds, bool kBatch>
-hipError_t Launch(const RenderParams& p, const LaunchShape& s, hipStream_t stream) {
+const void* RenderFn(const LaunchShape& s) {
   auto fn = kBatch ? BatchRenderKernel<kFast, kCount>
             : (!kLds && s.cacheOps > 0)
                 ? (s.block < 1024 ? RenderKernel<kFast, kCount, false, true, true>
                                   : RenderKernel<kFast, kCount, false, false, true>)
                 : (s.block < 1024 ? RenderKernel<kFast, kCount, kLds, true> : RenderKernel<kFast, kCount, kLds, false>);
-  hipError_t e = AllowLds(reinterpret_cast<const void*>(fn), s.lds);
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(fn, dim3(s.grid), dim3(s.block), s.lds, stream, p);
-  e = hipGetLastError();
-  if (e != hipSuccess || p.budget <= 0) return e;
-  // the heavy rays the first kernel handed over
-  auto coop = CoopKernel<kFast, kCount, kBatch>;
-  const size_t lds = CoopLaunchLds(p);
-  e = AllowLds(reinterpret_cast<const void*>(coop), lds);
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(coop, dim3(p.coopWaves), dim3(64), lds, stream, p);
-  return hipGetLastError();
+  return reinterpret_cast<const void*>(fn);
+}
+
+template <bool kFast, bool kCount>
+const void* RenderFn(const RenderParams& p, const LaunchShape& s) {
+  if (p.numJobs > 0) return RenderFn<kFast, kCount, false, true>(s);
+  return s.sceneInLds ? RenderFn<kFast, kCount, true, false>(s) : RenderFn<kFast, kCount, false, false>(s);
+}
+
+template <bool kFast, bool kCount>
+const void* CoopFn(const RenderParams& p) {
+  return p.numJobs > 0 ? reinterpret_cast<const void*>(CoopKernel<kFast, kCount, true>)
+                       : reinterpret_cast<const void*>(CoopKernel<kFast, kCount, false>);
 }
 
 struct DeviceLimits {
@@ -2297,18 +2419,50 @@ hipError_t ChooseShape(int32_t depthIn, size_t sceneBytes, const LaunchConfig& c
   return hipSuccess;
 }
 
-hipError_t LaunchRender(const RenderParams& p, const LaunchConfig& cfg, const LaunchShape& s, hipStream_t stream) {
+KernelLaunch MainLaunch(const RenderParams& p, const LaunchConfig& cfg, const LaunchShape& s) {
   const bool fast = cfg.mode == Mode::kFast;
-  if (p.numJobs > 0) {
-    if (fast) return cfg.count ? Launch<true, true, false, true>(p, s, stream) : Launch<true, false, false, true>(p, s, stream);
-    return cfg.count ? Launch<false, true, false, true>(p, s, stream) : Launch<false, false, false, true>(p, s, stream);
+  if (p.tileSlots > 0) {
+    const bool groups = p.tileGroups != 0;
+    auto tile = p.numJobs > 0 ? (groups ? TileKernel<true, true, true> : TileKernel<true, true, false>)
+                              : (groups ? TileKernel<true, false, true> : TileKernel<true, false, false>);
+    const void* fn = reinterpret_cast<const void*>(tile);
+    return KernelLaunch{fn, static_cast<uint32_t>(std::max(p.numTiles, 1)), 64, TileLds(p.tileSlots, p.stackSlots)};
   }
-  if (s.sceneInLds) {
-    if (fast) return cfg.count ? Launch<true, true, true, false>(p, s, stream) : Launch<true, false, true, false>(p, s, stream);
-    return cfg.count ? Launch<false, true, true, false>(p, s, stream) : Launch<false, false, true, false>(p, s, stream);
+  const void* fn = fast ? (cfg.count ? RenderFn<true, true>(p, s) : RenderFn<true, false>(p, s))
+                        : (cfg.count ? RenderFn<false, true>(p, s) : RenderFn<false, false>(p, s));
+  return KernelLaunch{fn, static_cast<uint32_t>(s.grid), static_cast<uint32_t>(s.block), s.lds};
+}
+
+KernelLaunch CoopLaunch(const RenderParams& p, const LaunchConfig& cfg) {
+  if (p.budget <= 0) return KernelLaunch{};
+  const bool fast = cfg.mode == Mode::kFast;
+  const void* fn = fast ? (cfg.count ? CoopFn<true, true>(p) : CoopFn<true, false>(p))
+                        : (cfg.count ? CoopFn<false, true>(p) : CoopFn<false, false>(p));
+  return KernelLaunch{fn, p.coopWaves, 64, CoopLaunchLds(p)};
+}
+
+hipError_t LaunchRender(const RenderParams& p, const LaunchConfig& cfg, const LaunchShape& s, hipStream_t stream) {
+  // the frame, then the heavy rays the first kernel handed over
+  for (const KernelLaunch& k : {MainLaunch(p, cfg, s), CoopLaunch(p, cfg)}) {
+    if (!k.fn) continue;
+    hipError_t e = AllowLds(k.fn, k.lds);
+    if (e != hipSuccess) return e;
+    void* args[1] = {const_cast<RenderParams*>(&p)};
+    e = hipLaunchKernel(k.fn, dim3(k.grid), dim3(k.block), args, k.lds, stream);
+    if (e != hipSuccess) return e;
   }
-  if (fast) return cfg.count ? Launch<true, true, false, false>(p, s, stream) : Launch<true, false, false, false>(p, s, stream);
-  return cfg.count ? Launch<false, true, false, false>(p, s, stream) : Launch<false, false, false, false>(p, s, stream);
+  return hipSuccess;
+}
+
+void PlanTiles(const LaunchConfig& cfg, bool groups, RenderParams* p) {
+  p->tileSlots = 0;
+  if (!cfg.tiles || cfg.mode != Mode::kFast || cfg.count) return;
+  const DeviceLimits* l = CurrentLimits();
+  if (!l || l->cus <= 0) return;
+  const int32_t slots = groups ? kTileSlots : kTilePlainSlots;
+  if (TileLds(slots, p->stackSlots) + kStaticLds > l->ldsPerCu || p->numTiles > kMaxTileGrid) return;
+  p->tileSlots = slots;
+  p->tileGroups = groups ? 1 : 0;
 }
 
 }  // namespace csgray

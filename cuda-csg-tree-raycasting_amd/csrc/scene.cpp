@@ -448,19 +448,21 @@ FlatScene Flatten(const CSGTree& tree) {
       const size_t first = f.walkOps.size();
       for (size_t c0 = 0; c0 < members.size(); c0 += kGroupChunk) {
         Box cb = tight[members[c0]];
+        bool out = !inside[members[c0]];
         for (size_t i = c0 + 1; i < std::min(members.size(), c0 + kGroupChunk); i++) {
+          out |= !inside[members[i]];
           for (int a = 0; a < 3; a++) {
             cb.lo[a] = std::min(cb.lo[a], tight[members[i]].lo[a]);
             cb.hi[a] = std::max(cb.hi[a], tight[members[i]].hi[a]);
           }
         }
         f.walkOps.push_back(F4{cb.lo[0], cb.lo[1], cb.lo[2], cb.hi[0]});
-        f.walkOps.push_back(F4{cb.hi[1], cb.hi[2], 0.0f, 0.0f});
+        f.walkOps.push_back(F4{cb.hi[1], cb.hi[2], 0.0f, bits(out ? 1u : 0u)});
       }
       for (const int32_t m : members) {
         const Box& b = tight[m];
         f.walkOps.push_back(F4{b.lo[0], b.lo[1], b.lo[2], b.hi[0]});
-        f.walkOps.push_back(F4{b.hi[1], b.hi[2], bits(desc(m)), 0.0f});
+        f.walkOps.push_back(F4{b.hi[1], b.hi[2], bits(desc(m)), bits(inside[m] ? 0u : 1u)});
         if (tree.nodes[m].primitiveIdx == -1) {
           F4& w = f.walkOps[4 * static_cast<size_t>(opIndex[m]) + 3];
           uint32_t tw;
@@ -474,6 +476,10 @@ FlatScene Flatten(const CSGTree& tree) {
       std::memcpy(&tw, &w.z, 4);
       w = F4{bits(static_cast<uint32_t>(first)), bits(static_cast<uint32_t>(members.size())), bits(tw | kGroupFlag),
              w.w};
+      if (members.size() >= static_cast<size_t>(kTileGroup)) {
+        if (f.tileOps.empty()) f.tileOps = f.ivOps;
+        f.tileOps[4 * static_cast<size_t>(gi) + 3] = w;
+      }
       f.unionGroups++;
     }
   }

@@ -85,10 +85,11 @@ struct CSGTree {
 // group's record holds bits(first chunk record, as a float4 index into
 // walkOps), bits(member count), type | right<<8 | kGroupFlag, parent.  After
 // the operator records, each group has one chunk record per kGroupChunk
-// members, (lo.x, lo.y, lo.z, hi.x), (hi.y, hi.z, 0, 0), the box around
+// members, (lo.x, lo.y, lo.z, hi.x), (hi.y, hi.z, 0, out), the box around
 // those members, and then one record per member,
-//   (lo.x, lo.y, lo.z, hi.x), (hi.y, hi.z, bits(desc), 0),
-// with its culling box, the members ordered by recursive median splits of
+//   (lo.x, lo.y, lo.z, hi.x), (hi.y, hi.z, bits(desc), out),
+// with its culling box (out = bits(1) where a primitive of it leaves its
+// box, else 0), the members ordered by recursive median splits of
 // their boxes' centres (so that a chunk's members lie close together); a member that is an
 // operator names the group as its parent (as a left child).  A larger Union
 // subtree stays binary at the top and its Union children are tried as
@@ -109,6 +110,10 @@ struct FlatScene {
   // The interval walk's records: ivOps with each Union group flattened, then
   // the groups' member records (layout below); empty without operators.
   std::vector<F4> walkOps;
+  // The tile kernel's operator records: ivOps with the Union groups of at
+  // least kTileGroup members flattened (their chunk and member records are
+  // walkOps'); empty where there is none.
+  std::vector<F4> tileOps;
   int32_t unionGroups = 0;  // Union groups flattened in walkOps
   uint32_t rootDesc = 0;
   int32_t nNodes = 0, nOps = 0, nPrims = 0, opDepth = 0;
@@ -118,6 +123,7 @@ struct FlatScene {
 
 constexpr uint32_t kGroupFlag = 0x200u;    // type word bit of a flattened Union group (walkOps)
 constexpr int32_t kMaxGroupMembers = 1024;  // a group's members are tested 64 a round by one wave
+constexpr int32_t kTileGroup = 24;          // smallest group the tile kernel takes flattened
 constexpr int32_t kGroupChunk = 4;          // members under one chunk box
 
 constexpr int32_t kMaxNodes = 65535;       // 16-bit node links
