@@ -195,6 +195,10 @@ void PrepareCoop(const LaunchConfig& cfg, int32_t maxOps, int32_t maxLeaves, boo
   p->budget = 0;
   PlanTiles(cfg, anyGroups, p);
   if (!heavy) return;
+  // Trees whose crossings always fit the tile kernel's lists, two a primitive,
+  // leave a few rays in millions (ties), which a lane finishes in at most a
+  // microsecond an operator; a cooperative launch, found empty, takes 4 us.
+  if (2 * (maxOps + 1) <= p->tileSlots) return;
   const bool lists = CoopLists(cfg, anyInBoxes);
   const CoopPlan c = PlanCoop(cfg, maxOps, maxLeaves, lists);
   if (c.budget <= 0) return;
