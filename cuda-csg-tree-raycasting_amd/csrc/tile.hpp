@@ -34,7 +34,13 @@
 //     Operators are re-entered at crossing times of their own or their
 //     ancestors' results only, so the ray is exact unless one of these lists
 //     has a crossing in [b, x): the zone, kept with the list as one interval
-//     around all the zones in it and tested at every operator above;
+//     around all the zones in it and tested at every operator above.  With
+//     one at t, that list is sure up to and including t, and what its next
+//     crossing is depends on when the machine asks.  So the operator above is
+//     sure up to its last crossing at or before t, if it has one, and so on
+//     to the root, whose first crossing is the answer if it is still sure
+//     (most zones lie on the far side of what the ray hits).  A mixed tree of
+//     200 at 1023x1023 hands over 70 rays so, 2234 if any such list fails;
 //   * more crossings than the stack holds.
 // A subtree is skipped for lanes whose answer cannot depend on it: an
 // Intersection's or a Difference's right child where the left list is empty
@@ -556,6 +562,11 @@ __device__ __forceinline__ void TileTrace(const Job& jb, const RayF& r, uint64_t
   uint64_t zoneLevels = 0;                                // levels whose left list's zone is saved
   int limit = slots;    // rows the lists may take; those above hold saved zones
   bool zones = false;   // some lane has met a zone
+  // A list with a crossing in its zone at `sure`, its operator's level and
+  // whether some lane has one: what the machine finds beyond is in doubt.
+  float sure = __builtin_inff();
+  int sureLevel = 0;
+  bool doubts = false;
   uint64_t cutLists = 0;  // lanes with a list ended at a tie: their zones outlive an empty list
   // frames of the entered operators: lane i holds level i's
   uint32_t fOp = 0, fRight = 0, fMl = 0, fMh = 0, fRl = 0, fRh = 0;
@@ -600,18 +611,21 @@ __device__ __forceinline__ void TileTrace(const Job& jb, const RayF& r, uint64_t
     list.Put(n == 2, sp + 1, last);
     sp += n;
   };
-  // Fails the lanes of `mask` with a crossing of their current list (from
-  // `base` on) in its zone.
-  auto testZone = [&](uint64_t mask, int base) CSG_INLINE {
+  // Whether this lane, if in `mask`, has a crossing of its current list (from
+  // `base` on) in its zone, and the first such time.
+  auto inZone = [&](uint64_t mask, int base, float& at) CSG_INLINE {
     const bool has = ((mask & me) != 0) & (zhi > zlo);
-    if (__ballot(has) == 0) return;
     bool in = false;
+    if (__ballot(has) != 0) {
 #pragma unroll 1
-    for (int i = base; __ballot(has & (i < sp)) != 0; i++) {
-      const float t = __uint_as_float(EntryTime(list.Get(i)));
-      in |= has & (i < sp) & (t >= zlo) & (t < zhi);
+      for (int i = base; __ballot(has & (i < sp)) != 0; i++) {
+        const float t = __uint_as_float(EntryTime(list.Get(i)));
+        const bool here = has & (i < sp) & (t >= zlo) & (t < zhi);
+        at = here & !in ? t : at;
+        in |= here;
+      }
     }
-    dead |= __ballot(in);
+    return in;
   };
   // Saves the current zones with level d's pending list.
   auto saveZones = [&]() CSG_INLINE {
@@ -846,7 +860,32 @@ __device__ __forceinline__ void TileTrace(const Job& jb, const RayF& r, uint64_t
         const bool empty = on & (sp == base) & !cut & ((cutLists & me) == 0);
         zlo = empty ? __builtin_inff() : zlo;
         zhi = empty ? -__builtin_inff() : zhi;
-        testZone(M, base);
+        // the last crossing a child's doubt leaves sure; none of an empty
+        // list that the other child alone has emptied
+        bool low = false;
+        if (doubts) {
+          low = on & (sureLevel > d);
+          if (__ballot(low) != 0) {
+            float last = -1.0f;
+#pragma unroll 1
+            for (int i = base; __ballot(low & (i < sp)) != 0; i++) {
+              const float t = __uint_as_float(EntryTime(list.Get(i)));
+              last = low & (i < sp) & (t <= sure) ? t : last;
+            }
+            const bool clear = low & none & !cut;
+            dead |= __ballot(low & !clear & (last < 0.0f));
+            sure = low ? (clear ? __builtin_inff() : last) : sure;
+            sureLevel = low ? (clear ? 0 : d) : sureLevel;
+            low &= !clear;
+          }
+        }
+        float at = 0.0f;
+        const bool in = inZone(M, base, at);
+        doubts |= __ballot(in) != 0;
+        // (one doubt a lane: with another pending, of a list beside this one, it fails)
+        dead |= __ballot(in & !low & (sure < __builtin_inff()));
+        sure = in ? fminf(sure, at) : sure;
+        sureLevel = in ? d : sureLevel;
       }
       state = kTileReturn;
     } else if (kGroups && state == kTileGroup) {
@@ -934,7 +973,11 @@ __device__ __forceinline__ void TileTrace(const Job& jb, const RayF& r, uint64_t
         }
       } else {
         const bool on = (M & me) != 0;
-        if (zones) testZone(M, base);
+        if (zones) {
+          float at;
+          const bool in = inZone(M, base, at);
+          dead |= __ballot(in | (on & (sureLevel > d)));
+        }
         int n = on ? sp - base : 0;
         // one member's (Enter, Exit) or lone Exit is a list already
         const bool sorts = (n > 2) | ((n == 2) & !(EntryBits(list.At(base)) & kEnter));
@@ -1002,11 +1045,8 @@ __device__ __forceinline__ uint32_t JobOfTile(const Job* jobs, uint32_t n, uint3
   return first + static_cast<uint32_t>(__popcll(__ballot(le2))) - 1u;
 }
 
-// Walks a tile's rays may take, and the least number of lanes with overflowing
-// lists worth stretches (fewer go the failed rays' way, as do all in a scene
-// whose primitives stay in their boxes: the cooperative kernel's interval
-// merge is faster there).
-constexpr int kTilePasses = 24, kTileMinFull = 8;
+// Walks a tile's rays may take.
+constexpr int kTilePasses = 24;
 // State-machine steps a failed ray takes in its lane before the cooperative
 // kernel gets it.  Most that fail on a tie end within 16, and a launch may
 // then have none to hand over; each step holds the whole wave up for about a
@@ -1089,10 +1129,13 @@ TileKernel(RenderParams p) {
     WaveSync();
     // The whole ray first.  Rays that fail in a scene with Union groups are
     // walked again through the tree as it is, where every comparison is the
-    // machine's own.  If many lanes' lists overflow, those again over
+    // machine's own.  Then the lanes whose lists overflow, again over
     // consecutive stretches of the ray (half its extent in the root's
     // children's boxes, halved while a list overflows, grown after each
-    // that fits, the last one open-ended), to its end.
+    // that fits, the last one open-ended), to its end: a large random tree's
+    // frame takes 10.1 ms so, 10.9 ms with fewer than 8 such lanes handed over.
+    // (Where all primitives stay in their boxes the cooperative kernel merges
+    // intervals, which is faster: the 512-sphere frame 209 us, 306 so.)
     uint64_t todo = active, over = 0;
     float ts = 0.0f, te = __builtin_inff(), w = 0.0f, end = 0.0f;
     const float4* ops = jb.sc.tileOps;
@@ -1114,7 +1157,7 @@ TileKernel(RenderParams p) {
         }
         fail |= failed;
         todo = over;
-        if (jb.sc.conservative || __popcll(over) < kTileMinFull) break;
+        if (jb.sc.conservative || over == 0) break;
         const U32x16 o = ScalarRecord(jb.sc.tileOps, 0);
         float nL, xL, nR, xR;
         Slab<true>(r, __uint_as_float(o[0]), __uint_as_float(o[1]), __uint_as_float(o[2]), __uint_as_float(o[4]),
