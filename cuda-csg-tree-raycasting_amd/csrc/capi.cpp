@@ -703,7 +703,7 @@ csg_status csg_render_ex(const csg_scene* s, const csg_camera* cam, const csg_li
     const csg_status hsd = HeavyFor(dev, hs, &heavy);
     if (hsd != CSG_OK) return hsd;
   }
-  cfg.tiles = cfg.tiles && cfg.sceneInLds == -1 && !p.tileOrder && TilesPay(s, p.numTiles);
+  cfg.tiles = cfg.tiles && cfg.sceneInLds == -1 && !p.tileOrder;
   PrepareCoop(cfg, s->dev.nOps, s->dev.opLeaves, s->dev.conservative != 0, HasTileGroups(s), heavy, shape, &p);
   e = csgray::LaunchRender(p, cfg, shape, hs);
   if (e != hipSuccess) return FailHip(e, "render launch");

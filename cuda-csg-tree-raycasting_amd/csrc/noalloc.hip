@@ -114,7 +114,7 @@ extern "C" csg_status csg_render_noalloc(const csg_scene* s, const csg_camera* c
   if (ss != CSG_OK) return ss;
   p.queue = reinterpret_cast<uint32_t*>(base);
   uint2* heavy = reinterpret_cast<uint2*>(base + kQueueRegion);
-  cfg.tiles = cfg.tiles && cfg.sceneInLds == -1 && !p.tileOrder && TilesPay(s, p.numTiles);
+  cfg.tiles = cfg.tiles && cfg.sceneInLds == -1 && !p.tileOrder;
   PrepareCoop(cfg, s->dev.nOps, s->dev.opLeaves, s->dev.conservative != 0, HasTileGroups(s),
               cfg.budget >= 0 ? heavy : nullptr, shape, &p);
   p.resumeBytes = static_cast<uint32_t>(kNoAllocResumeBytes);

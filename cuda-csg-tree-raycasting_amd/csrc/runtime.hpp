@@ -33,17 +33,6 @@ size_t SceneBytes(const csg_scene* s);
 // Whether the tile kernel takes Union groups of the scene.
 inline bool HasTileGroups(const csg_scene* s) { return s->dev.tileOps != s->dev.ivOps; }
 
-// Whether a launch of this one scene and `tiles` 8x8 tiles classifies whole
-// tiles.  In a scene with a primitive that leaves its box some rays always go
-// the cooperative kernel's way, which costs such a launch 15-30 us after its
-// tiles; a small tree's per-lane frame is over by then.  Mixed trees of 12, 24,
-// 32 and 40 leaves at 640x360, per lane and by tiles: 33 and 57, 62 and 82, 66
-// and 92, 101 and 101 us; of 12 and 24 at 1920x1080: 77 and 71, 111 and 114,
-// of 24 at 3840x2160: 320 and 218; of 6 at 640x360: 27 and 21.
-inline bool TilesPay(const csg_scene* s, int64_t tiles) {
-  return s->dev.conservative != 0 || s->dev.nOps < 8 || s->dev.nOps >= 40 || tiles >= 32000;
-}
-
 // Validates one job and fills its device descriptor; `tileBase` is its first
 // queue index within the launch.
 csg_status BuildJob(const csg_scene* s, const csg_camera* cam, const csg_light* light, const csg_phong* phong,
