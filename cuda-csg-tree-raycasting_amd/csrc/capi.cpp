@@ -193,12 +193,12 @@ int32_t DefaultCoopGraceMille(int64_t waves, int64_t tiles, bool batched, bool l
 void PrepareCoop(const LaunchConfig& cfg, int32_t maxOps, int32_t maxLeaves, bool anyInBoxes, bool anyGroups,
                  uint2* heavy, const LaunchShape& shape, RenderParams* p) {
   p->budget = 0;
-  PlanTiles(cfg, anyGroups, p);
+  PlanTiles(cfg, anyGroups, maxOps, p);
   if (!heavy) return;
   // Trees whose crossings always fit the tile kernel's lists, two a primitive,
   // leave a few rays in millions (ties), which a lane finishes in at most a
   // microsecond an operator; a cooperative launch, found empty, takes 4 us.
-  if (2 * (maxOps + 1) <= p->tileSlots) return;
+  if (p->tileSlots > 0 && 2 * (maxOps + 1) <= kTilePlainSlots) return;
   const bool lists = CoopLists(cfg, anyInBoxes);
   const CoopPlan c = PlanCoop(cfg, maxOps, maxLeaves, lists);
   if (c.budget <= 0) return;

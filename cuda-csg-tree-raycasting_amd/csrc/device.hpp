@@ -152,11 +152,25 @@ hipError_t ChooseShape(int32_t depth, size_t sceneBytes, const LaunchConfig& cfg
 // Compute units, LDS bytes per workgroup and per CU of the current device.
 hipError_t DeviceShapeLimits(int* computeUnits, size_t* ldsPerBlock, size_t* ldsPerCu = nullptr);
 
-// Tile kernel (tile.hpp): entries of a lane's list stack and waves a CU holds,
-// with Union groups and without, and one wave's LDS for trees of `depth`
-// operator levels.
+// Tile kernel (tile.hpp): entries of a lane's list stack, with Union groups
+// and without.  Fewer leave room for more waves, more hand over fewer rays:
+// the 512-sphere frame takes 215, 210 and 194 us with 24, 26 and 28, but with
+// 28 next to none of its rays go to the cooperative kernel, as callers that
+// watch its counter expect of that frame.
 constexpr int32_t kTileSlots = 26, kTilePlainSlots = 16;
+// Exact mode, trees of fewer than kTileExactSmall operators and others.  At
+// 640x360, 24 and 40 slots: unions of 400 541 and 579 us, trees of 200 373 and
+// 378; 512 spheres taken from a cube 973 and 781 us, 1500 4754 and 3975.
+constexpr int32_t kTileExactSmall = 448, kTileExactSmallSlots = 24, kTileExactSlots = 40;
+// Exact mode walks every operator whose boxes a tile's rays hit, at two slab
+// tests with six divisions each, for all 64 rays: the larger the tree, the
+// fewer of them need it.  Per lane and by tiles, 640x360: mixed trees of 200
+// and 800 974 and 377, 3237 and 1981 us; 512 and 1500 spheres taken from a cube
+// 910 and 788, 5447 and 4027 us; unions of 400 and 2000 772 and 569, 3646 and
+// 3994 us; of 4095 at 320x180 5740 and 9002 us.
+constexpr int32_t kTileExactOps = 1750;
 constexpr int32_t kMaxTileGrid = 0x3FFFFFF;  // a grid has fewer than 2^32 threads
+// One wave's LDS for trees of `depth` operator levels.
 constexpr size_t TileLds(int32_t slots, int32_t depth) {
   const size_t bytes = 512 * static_cast<size_t>(slots + 2) + 64 + 144 + 64 * static_cast<size_t>(depth > 0 ? depth : 1);
   return (bytes + 15) & ~static_cast<size_t>(15);
@@ -164,8 +178,8 @@ constexpr size_t TileLds(int32_t slots, int32_t depth) {
 
 // Fills the tile kernel's fields of `p` (numTiles and stackSlots set):
 // tileSlots stays 0 where it does not apply.  `groups`: some scene of the
-// launch has Union groups in its tileOps.
-void PlanTiles(const LaunchConfig& cfg, bool groups, RenderParams* p);
+// launch has Union groups in its tileOps; `ops`: the most operators of one.
+void PlanTiles(const LaunchConfig& cfg, bool groups, int32_t ops, RenderParams* p);
 
 // One kernel of a launch: the kernel that renders the frame, and the
 // cooperative one (fn null when none follows).

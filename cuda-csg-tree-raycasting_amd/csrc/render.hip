@@ -2425,6 +2425,7 @@ KernelLaunch MainLaunch(const RenderParams& p, const LaunchConfig& cfg, const La
     const bool groups = p.tileGroups != 0;
     auto tile = p.numJobs > 0 ? (groups ? TileKernel<true, true, true> : TileKernel<true, true, false>)
                               : (groups ? TileKernel<true, false, true> : TileKernel<true, false, false>);
+    if (!fast) tile = p.numJobs > 0 ? TileKernel<false, true, false> : TileKernel<false, false, false>;
     const void* fn = reinterpret_cast<const void*>(tile);
     return KernelLaunch{fn, static_cast<uint32_t>(std::max(p.numTiles, 1)), 64, TileLds(p.tileSlots, p.stackSlots)};
   }
@@ -2454,12 +2455,14 @@ hipError_t LaunchRender(const RenderParams& p, const LaunchConfig& cfg, const La
   return hipSuccess;
 }
 
-void PlanTiles(const LaunchConfig& cfg, bool groups, RenderParams* p) {
+void PlanTiles(const LaunchConfig& cfg, bool groups, int32_t ops, RenderParams* p) {
   p->tileSlots = 0;
-  if (!cfg.tiles || cfg.mode != Mode::kFast || cfg.count) return;
+  if (!cfg.tiles || cfg.count || (cfg.mode == Mode::kExact && ops > kTileExactOps)) return;
   const DeviceLimits* l = CurrentLimits();
   if (!l || l->cus <= 0) return;
-  const int32_t slots = groups ? kTileSlots : kTilePlainSlots;
+  groups = groups && cfg.mode == Mode::kFast;  // (their boxes are the fast mode's)
+  const int32_t exact = ops < kTileExactSmall ? kTileExactSmallSlots : kTileExactSlots;
+  const int32_t slots = cfg.mode == Mode::kExact ? exact : groups ? kTileSlots : kTilePlainSlots;
   if (TileLds(slots, p->stackSlots) + kStaticLds > l->ldsPerCu || p->numTiles > kMaxTileGrid) return;
   p->tileSlots = slots;
   p->tileGroups = groups ? 1 : 0;

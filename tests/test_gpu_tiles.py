@@ -26,10 +26,12 @@ def _mixed(n, seed):
     return "\n".join(S.random_ops_balanced(rng, leaves)) + "\n"
 
 
-# A Union group is walked by its boxes from 24 members on.
 SCENES = {
+    # a Union group is walked by its boxes from 24 members on
     "sphere": lambda: S.sphere((0, 0, 0), "C8503C", 0.9) + "\n",
-    **{f"cheese{n}": lambda n=n: S.cheese(n, seed=n) for n in (1, 22, 23, 24, 25, 64, 65, 512)},
+    # Exact mode has longer lists from 448 operators on, and takes trees of up to
+    # 1750 by tiles.
+    **{f"cheese{n}": lambda n=n: S.cheese(n, seed=n) for n in (1, 22, 23, 24, 25, 64, 65, 447, 448, 512, 1750, 1751)},
     **{f"mixed{n}": lambda n=n: _mixed(n, n) for n in (2, 8, 9, 39, 40, 41, 128)},
     "difference64": lambda: deep.left_deep_difference(64, seed=3),
     "union64": lambda: deep.right_deep_union(64, seed=3),
@@ -41,16 +43,17 @@ SCENES = {
 }
 
 
+@pytest.mark.parametrize("mode", [C.MODE_FAST, C.MODE_EXACT], ids=["fast", "exact"])
 @pytest.mark.parametrize("name", list(SCENES))
-def test_tiles_equal_the_state_machine(gpu, name):
+def test_tiles_equal_the_state_machine(gpu, name, mode):
     scene = C.Scene(SCENES[name]())
     light, phong = C.light((0.4, 0.7, 0.6)), C.phong(0.2, 0.7, 0.3, 16.0)
     eyes = [(2.2, 1.3, 2.9), (0.05, 0.02, 0.04), (0.0, 0.0, 4.0)]  # outside, inside the solid, along an axis
     for (w, h, samples), eye in zip([(2, 2, 1), (8, 8, 1), (65, 33, 1), (130, 71, 3), (320, 200, 1)], eyes + eyes[:2]):
         cam = C.camera_look_at(eye, (0.0, 0.01, 0.0), 55)
         print(f"[case] {name} {w}x{h} samples {samples}", flush=True)
-        got = scene.render(cam, light, phong, w, h, samples=samples, seed=5)
-        ref = scene.render(cam, light, phong, w, h, samples=samples, seed=5, coop=-1)
+        got = scene.render(cam, light, phong, w, h, samples=samples, seed=5, mode=mode)
+        ref = scene.render(cam, light, phong, w, h, samples=samples, seed=5, mode=mode, coop=-1)
         torch.cuda.synchronize()
         for key in ("rgba", "depth", "prim_id", "flags"):
             a, b = got[key].cpu().numpy(), ref[key].cpu().numpy()
