@@ -1062,6 +1062,17 @@ constexpr int kTilePasses = 24;
 // 16 225, 48 227 us; the 512-sphere frame (lists overflow): 236, 243, 259 us.
 constexpr int kTileSteps = 16;
 
+// Whether the cooperative kernel has been handed fewer rays than it has waves.
+// Such rays are traced side by side, where a tile's stretches follow one
+// another: a union of 1143 at 292x164 takes 427 to 637 us so, 630 to 1276 with
+// stretches alone (30 rays overflow a list), at 1280x720 420 to 578 and 507 to
+// 1034; of 4095 at 1920x1080, 4 samples, 8.1 and 7.7 ms (190 ms with all rays
+// handed over).
+__device__ __forceinline__ bool HandsOverFew(const RenderParams& p) {
+  const uint32_t n = __hip_atomic_load(p.queue + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return p.heavyCap != 0 && __builtin_amdgcn_readfirstlane(n) < p.coopWaves;
+}
+
 // One wave, one tile.  kGroups: some scene of the launch has Union groups;
 // without, the code is half as long and takes half the registers, and shorter
 // lists do (4 waves a SIMD instead of 2).  Workgroups come from the hardware's
@@ -1135,15 +1146,17 @@ TileKernel(RenderParams p) {
     lds.bundle[2] = make_float4(bundle.c[2], bundle.k[0], bundle.k[1], bundle.k[2]);
     lds.bundle[3] = make_float4(scale.lo, scale.hi, 0.0f, 0.0f);
     WaveSync();
-    // The whole ray first.  Rays that fail in a scene with Union groups are
-    // walked again through the tree as it is, where every comparison is the
-    // machine's own.  Then the lanes whose lists overflow, again over
+    // The whole ray first.  Rays that fail, on a tie in a Union group for
+    // the most part, go to the cooperative kernel; without one, they are walked
+    // again through the tree as it is, where every comparison is the
+    // machine's own (a walk of all 512 spheres for one ray kept the frame of
+    // some views 700 us instead of 200).  Then the lanes whose lists overflow,
+    // unless the cooperative kernel has room (HandsOverFew), again over
     // consecutive stretches of the ray (half its extent in the root's
     // children's boxes, halved while a list overflows, grown after each
-    // that fits, the last one open-ended), to its end: a large random tree's
-    // frame takes 10.1 ms so, 10.9 ms with fewer than 8 such lanes handed over.
-    // (Where all primitives stay in their boxes the cooperative kernel merges
-    // intervals, which is faster: the 512-sphere frame 209 us, 306 so.)
+    // that fits, the last one open-ended), to its end.  (Where all primitives
+    // stay in their boxes the cooperative kernel merges intervals, which is
+    // always faster: the 512-sphere frame 209 us, 306 with stretches.)
     uint64_t todo = active, over = 0;
     float ts = 0.0f, te = __builtin_inff(), w = 0.0f, end = 0.0f;
     const float4* ops = jb.sc.tileOps;
@@ -1157,7 +1170,7 @@ TileKernel(RenderParams p) {
         h.t = mine ? first.t : h.t;
         h.bits = mine ? first.bits : h.bits;
         over |= full;
-        if (stage == 0 && failed != 0 && ops != jb.sc.ops) {
+        if (stage == 0 && failed != 0 && ops != jb.sc.ops && p.heavyCap == 0) {
           ops = jb.sc.ops;
           todo = failed;
           stage = 1;
@@ -1165,7 +1178,7 @@ TileKernel(RenderParams p) {
         }
         fail |= failed;
         todo = over;
-        if (jb.sc.conservative || over == 0) break;
+        if (jb.sc.conservative || over == 0 || HandsOverFew(p)) break;
         const U32x16 o = ScalarRecord(jb.sc.tileOps, 0);
         float nL, xL, nR, xR;
         Slab<true>(r, __uint_as_float(o[0]), __uint_as_float(o[1]), __uint_as_float(o[2]), __uint_as_float(o[4]),
