@@ -193,7 +193,7 @@ int32_t DefaultCoopGraceMille(int64_t waves, int64_t tiles, bool batched, bool l
 void PrepareCoop(const LaunchConfig& cfg, int32_t maxOps, int32_t maxLeaves, bool anyInBoxes, bool anyGroups,
                  uint2* heavy, const LaunchShape& shape, RenderParams* p) {
   p->budget = 0;
-  PlanTiles(cfg, anyGroups, maxOps, p);
+  PlanTiles(cfg, anyGroups, anyInBoxes, maxOps, p);
   if (!heavy) return;
   // Trees whose crossings always fit the tile kernel's lists, two a primitive,
   // leave a few rays in millions (ties), which a lane finishes in at most a

@@ -158,17 +158,23 @@ hipError_t DeviceShapeLimits(int* computeUnits, size_t* ldsPerBlock, size_t* lds
 // 28 next to none of its rays go to the cooperative kernel, as callers that
 // watch its counter expect of that frame.
 constexpr int32_t kTileSlots = 26, kTilePlainSlots = 16;
-// Exact mode, trees of fewer than kTileExactSmall operators and others.  At
+// Exact mode, trees of fewer than kTileLargeOps operators and others.  At
 // 640x360, 24 and 40 slots: unions of 400 541 and 579 us, trees of 200 373 and
 // 378; 512 spheres taken from a cube 973 and 781 us, 1500 4754 and 3975.
-constexpr int32_t kTileExactSmall = 448, kTileExactSmallSlots = 24, kTileExactSlots = 40;
-// Exact mode walks every operator whose boxes a tile's rays hit, at two slab
-// tests with six divisions each, for all 64 rays: the larger the tree, the
-// fewer of them need it.  Per lane and by tiles, 640x360: mixed trees of 200
-// and 800 974 and 377, 3237 and 1981 us; 512 and 1500 spheres taken from a cube
-// 910 and 788, 5447 and 4027 us; unions of 400 and 2000 772 and 569, 3646 and
-// 3994 us; of 4095 at 320x180 5740 and 9002 us.
-constexpr int32_t kTileExactOps = 1750;
+constexpr int32_t kTileLargeOps = 448, kTileExactSmallSlots = 24, kTileExactSlots = 40;
+// A tile's walk of a large tree is one long chain, which few tiles do not
+// hide; the per-lane kernel and a wave a heavy ray are faster for them.  Fast
+// mode takes tiles from kTileLargeTiles on (per lane and by tiles: 500 spheres
+// taken from a cube, 64 tiles 99 and 257 us, 475 162 and 170, 2394 204 and 139;
+// 1500, 475 tiles 226 and 411 us, 2394 787 and 653; a union of 4095, 475 tiles
+// 3110 and 7570 us, 2394 7510 and 4885).  Exact mode, which has no groups, from
+// 5 a operator on (a union of 700, 950 tiles 863 and 988 us, 4400 1313 and
+// 1035; of 1000, 4400 1400 and 1508, 14,400 2437 and 1821; of 2000, 3600 3646
+// and 3669, 14,400 10434 and 4699; of 400, 100 tiles 754 and 669).
+// Where the cooperative kernel merges intervals, middle-sized trees need a few
+// hundred too: 128 spheres, 64 tiles 89 and 68 us; 256, 144 tiles 95 and 123, 475
+// 147 and 82.
+constexpr int32_t kTileLargeTiles = 2000, kTileMiddleOps = 192, kTileMiddleTiles = 300;
 constexpr int32_t kMaxTileGrid = 0x3FFFFFF;  // a grid has fewer than 2^32 threads
 // One wave's LDS for trees of `depth` operator levels.
 constexpr size_t TileLds(int32_t slots, int32_t depth) {
@@ -178,8 +184,9 @@ constexpr size_t TileLds(int32_t slots, int32_t depth) {
 
 // Fills the tile kernel's fields of `p` (numTiles and stackSlots set):
 // tileSlots stays 0 where it does not apply.  `groups`: some scene of the
-// launch has Union groups in its tileOps; `ops`: the most operators of one.
-void PlanTiles(const LaunchConfig& cfg, bool groups, int32_t ops, RenderParams* p);
+// launch has Union groups in its tileOps; `inBoxes`: all
+// primitives of some scene stay in their boxes; `ops`: the most operators of one.
+void PlanTiles(const LaunchConfig& cfg, bool groups, bool inBoxes, int32_t ops, RenderParams* p);
 
 // One kernel of a launch: the kernel that renders the frame, and the
 // cooperative one (fn null when none follows).

@@ -2455,14 +2455,17 @@ hipError_t LaunchRender(const RenderParams& p, const LaunchConfig& cfg, const La
   return hipSuccess;
 }
 
-void PlanTiles(const LaunchConfig& cfg, bool groups, int32_t ops, RenderParams* p) {
+void PlanTiles(const LaunchConfig& cfg, bool groups, bool inBoxes, int32_t ops, RenderParams* p) {
   p->tileSlots = 0;
-  if (!cfg.tiles || cfg.count || (cfg.mode == Mode::kExact && ops > kTileExactOps)) return;
+  const bool exact = cfg.mode == Mode::kExact;
+  const int64_t least = ops >= kTileLargeOps ? (exact ? 5 * int64_t{ops} : kTileLargeTiles)
+                        : !exact && inBoxes && ops >= kTileMiddleOps ? kTileMiddleTiles : 0;
+  if (!cfg.tiles || cfg.count || p->numTiles < least) return;
   const DeviceLimits* l = CurrentLimits();
   if (!l || l->cus <= 0) return;
-  groups = groups && cfg.mode == Mode::kFast;  // (their boxes are the fast mode's)
-  const int32_t exact = ops < kTileExactSmall ? kTileExactSmallSlots : kTileExactSlots;
-  const int32_t slots = cfg.mode == Mode::kExact ? exact : groups ? kTileSlots : kTilePlainSlots;
+  groups = groups && !exact;  // (their boxes are the fast mode's)
+  const int32_t slots = exact ? (ops < kTileLargeOps ? kTileExactSmallSlots : kTileExactSlots)
+                              : (groups ? kTileSlots : kTilePlainSlots);
   if (TileLds(slots, p->stackSlots) + kStaticLds > l->ldsPerCu || p->numTiles > kMaxTileGrid) return;
   p->tileSlots = slots;
   p->tileGroups = groups ? 1 : 0;

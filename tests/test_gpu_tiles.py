@@ -29,9 +29,9 @@ def _mixed(n, seed):
 SCENES = {
     # a Union group is walked by its boxes from 24 members on
     "sphere": lambda: S.sphere((0, 0, 0), "C8503C", 0.9) + "\n",
-    # Exact mode has longer lists from 448 operators on, and takes trees of up to
-    # 1750 by tiles.
-    **{f"cheese{n}": lambda n=n: S.cheese(n, seed=n) for n in (1, 22, 23, 24, 25, 64, 65, 447, 448, 512, 1750, 1751)},
+    # trees of 448 operators or more have longer lists in exact mode and go by
+    # tiles from 2000 tiles on in fast mode, 5 an operator in exact mode
+    **{f"cheese{n}": lambda n=n: S.cheese(n, seed=n) for n in (1, 22, 23, 24, 25, 64, 65, 447, 448, 512)},
     **{f"mixed{n}": lambda n=n: _mixed(n, n) for n in (2, 8, 9, 39, 40, 41, 128)},
     "difference64": lambda: deep.left_deep_difference(64, seed=3),
     "union64": lambda: deep.right_deep_union(64, seed=3),
@@ -49,7 +49,8 @@ def test_tiles_equal_the_state_machine(gpu, name, mode):
     scene = C.Scene(SCENES[name]())
     light, phong = C.light((0.4, 0.7, 0.6)), C.phong(0.2, 0.7, 0.3, 16.0)
     eyes = [(2.2, 1.3, 2.9), (0.05, 0.02, 0.04), (0.0, 0.0, 4.0)]  # outside, inside the solid, along an axis
-    for (w, h, samples), eye in zip([(2, 2, 1), (8, 8, 1), (65, 33, 1), (130, 71, 3), (320, 200, 1)], eyes + eyes[:2]):
+    for (w, h, samples), eye in zip([(2, 2, 1), (8, 8, 1), (65, 33, 1), (130, 71, 3), (320, 200, 1),
+                                   (397, 319, 1), (400, 320, 1), (400, 360, 1)], eyes + eyes + eyes[:2]):
         cam = C.camera_look_at(eye, (0.0, 0.01, 0.0), 55)
         print(f"[case] {name} {w}x{h} samples {samples}", flush=True)
         got = scene.render(cam, light, phong, w, h, samples=samples, seed=5, mode=mode)
