@@ -417,7 +417,7 @@ def main():
                         traffic = int(ln.split(":")[1])
         roofline = {"bound": "valu_fp32", "achieved": round(achieved, 3), "peak": PEAK_FP32_TFLOPS,
                     "unit": "TFLOP/s", "frac": round(achieved / PEAK_FP32_TFLOPS, 4), "traffic": traffic,
-                    "flops_per_ray": round(fpr, 1), "kernel": "render call (RenderKernel + CoopKernel)",
+                    "flops_per_ray": round(fpr, 1), "kernel": "render call (TileKernel + CoopKernel)",
                     "avg_kernel_ms": round(avg_kernel_ms, 4)}
 
     extra = {}

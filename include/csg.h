@@ -274,7 +274,8 @@ csg_status csg_batch_create(const csg_job* jobs, int32_t njobs, const csg_render
  * the graph's kernel nodes get new parameters. */
 csg_status csg_batch_update(csg_batch* batch, const csg_job* jobs, int32_t njobs, void* stream);
 csg_status csg_batch_launch(csg_batch* batch, void* stream);
-/* Times candidate launch shapes on the batch (workgroup 256/512/1024 lanes x
+/* Times candidate launch shapes on the batch (whole tiles, reported with the
+ * default `block`, or workgroups of 256/512/1024 lanes x
  * row-major/Morton tile walk x given/heaviest-first job order x LDS stack
  * depth: one launch whose stacks fit the deepest tree, or two depth classes
  * split at the depth that halves the batch's work (pixels x depth; failing
@@ -291,9 +292,11 @@ typedef struct csg_batch_tuning {
 csg_status csg_batch_autotune(csg_batch* batch, int32_t reps, void* stream, csg_batch_tuning* chosen);
 csg_status csg_batch_free(csg_batch* batch);
 
-/* Launch geometry csg_render_ex would use for this scene and options on the
+/* Launch geometry of the per-lane kernel for this scene and options on the
  * current device, for a large frame (no reference counterpart; for tests and
- * tuning).  A single-scene launch with the scene in LDS takes 1024-lane
+ * tuning).  csg_render_ex uses it when an option shapes it (block, placement,
+ * tile order, counters, hand-over, boxes) and for large trees in few tiles;
+ * otherwise a workgroup of one wave classifies each 8x8 tile.  A single-scene launch with the scene in LDS takes 1024-lane
  * workgroups when they fit, the scene has at least 256 operators and the frame
  * has an 8x8 tile for every wave of that grid; otherwise 512 lanes. */
 typedef struct csg_launch_info {
