@@ -242,6 +242,7 @@ void CSGTree::ConstructBVH() {
 
 FlatScene Flatten(const CSGTree& tree) {
   FlatScene f;
+  size_t inTileGroups = 0;  // members of the Union groups tileOps walks
   f.nNodes = static_cast<int32_t>(tree.nodes.size());
   f.nPrims = static_cast<int32_t>(tree.primitives.size());
   f.opDepth = tree.opDepth;
@@ -479,10 +480,16 @@ FlatScene Flatten(const CSGTree& tree) {
       if (members.size() >= static_cast<size_t>(kTileGroup)) {
         if (f.tileOps.empty()) f.tileOps = f.ivOps;
         f.tileOps[4 * static_cast<size_t>(gi) + 3] = w;
+        inTileGroups += members.size();
       }
       f.unionGroups++;
     }
   }
+  // Groups that hold few of a scene's primitives are not worth the kernel that
+  // walks them, which runs half as many waves and goes over a ray whose list
+  // overflows in stretches: mixed trees of 796 at 624x624 take 5.6 ms with it,
+  // 1.8 ms without, of 900 at 1280x720 4.9 and 2.8 ms.
+  if (4 * inTileGroups < static_cast<size_t>(f.nPrims)) f.tileOps.clear();
   return f;
 }
 
