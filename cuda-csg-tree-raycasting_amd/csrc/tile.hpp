@@ -26,7 +26,10 @@
 //     operator combines; in a Union group, whose members it pairs up in some
 //     order, two equal Enters or Exits of any members count;
 //   * in a Union group or a stretch, a primitive whose crossings are not
-//     (Enter, Exit) or a lone Exit;
+//     (Enter, Exit) or a lone Exit, and an operator in a Union group whose list
+//     is not a solid's (two Enters or two Exits in a row, or no Exit at its
+//     end, as a tie or a zone leaves it): the group counts the members a ray is
+//     inside of;
 //   * a tilted cylinder that leaves its box: the machine enters a primitive's
 //     operator only by its boxes, so re-entered at a tmin beyond the box's
 //     exit b it takes the cylinder for missed although its own exit x > b is
@@ -346,8 +349,9 @@ __device__ __forceinline__ int CombineSpecial(const TileList& l, int base, int n
 }
 
 // The union of the n <= S crossings from `base` on, in any order: sorted and
-// swept with a count of the members the ray is inside of.  Every list ends
-// outside, so the members it starts inside of are the surplus of Exits.
+// swept with a count of the members the ray is inside of.  Every member's list
+// alternates and ends with an Exit (NoSolid fails the rays of others), so the
+// members the ray starts inside of are the surplus of Exits.
 // False, with the entries sorted in place, when two have one time.
 template <int S>
 __device__ __forceinline__ bool Unite(const TileList& l, int base, int n, int& len) {
@@ -377,6 +381,20 @@ __device__ __forceinline__ bool Unite(const TileList& l, int base, int n, int& l
   }
   len = w - base;
   return true;
+}
+
+// Whether the list in rows [from, to) is not a solid's: two Enters or two Exits
+// in a row, or an Enter at its end.
+__device__ __forceinline__ bool NoSolid(const TileList& l, int from, int to) {
+  bool odd = false;
+  uint32_t bits = EntryBits(l.Get(from));
+#pragma unroll 1
+  for (int i = from; __ballot(i < to) != 0; i++) {
+    const uint32_t next = i + 1 < to ? EntryBits(l.Get(i + 1)) : kEnter;
+    odd |= (i < to) & (((bits ^ next) & kEnter) == 0);
+    bits = next;
+  }
+  return odd;
 }
 
 // The same from sorted entries in LDS with equal times among them: an Enter
@@ -709,6 +727,8 @@ __device__ __forceinline__ void TileTrace(const Job& jb, const RayF& r, uint64_t
         if (state == kTileRight) mR = ~uint64_t{0};  // (its right list was evaluated)
       }
       if (kGroups && state == kTileGroup) {
+        // (the member's list lies in rows [mid, sp))
+        dead |= __ballot(NoSolid(list, mid, sp));
         q = ScalarRecord(ops, 4 * X);
         // this member round again, past the member it left off at
         cr = static_cast<uint32_t>(mR) >> 8;
