@@ -192,7 +192,12 @@ int32_t DefaultCoopGraceMille(int64_t waves, int64_t tiles, bool batched, bool l
 
 void PrepareCoop(const LaunchConfig& cfg, int32_t maxOps, int32_t maxLeaves, bool anyInBoxes, bool anyGroups,
                  uint2* heavy, const LaunchShape& shape, RenderParams* p) {
+  // (a launch without a cooperative kernel must not hand rays over, whatever
+  // an earlier launch left in `p`)
   p->budget = 0;
+  p->heavy = nullptr;
+  p->heavyCap = 0;
+  p->coopWaves = 0;
   PlanTiles(cfg, anyGroups, anyInBoxes, maxOps, p);
   if (!heavy) return;
   // Trees whose crossings always fit the tile kernel's lists, two a primitive,
@@ -739,10 +744,10 @@ csg_status csg_render_batch(const csg_job* jobs, int32_t njobs, const csg_render
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return FailHip(e, "hipGetDevice");
   const hipStream_t hs = static_cast<hipStream_t>(stream);
-  csgray::RenderParams p{};
   int32_t depth = 1;
   int64_t base = 0;
   for (int32_t start = 0; start < njobs; start += csgray::kMaxBatchJobs) {
+    csgray::RenderParams p{};
     const int32_t n = std::min(njobs - start, csgray::kMaxBatchJobs);
     std::vector<csgray::Job> host(static_cast<size_t>(n));
     base = 0;

@@ -1,0 +1,63 @@
+"""Batches of several launches (1024 jobs each) through the tile kernel: a
+launch whose trees need no cooperative kernel hands no rays over, whatever the
+launch before it did."""
+import numpy as np
+import pytest
+import torch
+import csgray as C
+from csgray import scenes as S
+
+pytestmark = pytest.mark.gpu
+
+KEYS = ("rgba", "depth", "prim_id", "flags")
+LIGHT, PHONG = (0.4, 0.7, 0.6), (0.2, 0.7, 0.3, 16.0)
+
+
+def _flush_cubes(seed=174):
+    """Eight cubes with many flush faces under seven operators: some rays meet ties they must trace to the end."""
+    rng = np.random.default_rng(seed)
+    cubes = [S.cube(tuple(float(v) * 0.5 for v in rng.integers(-2, 3, 3)), "C85A5A", float(rng.integers(1, 4)) * 0.5)
+             for _ in range(8)]
+    return "\n".join(S.random_ops_balanced(rng, cubes)) + "\n"
+
+
+def test_a_later_launch_of_small_trees_finishes_its_rays(gpu):
+    small = C.Scene(_flush_cubes())
+    # nine primitives, out of sight: a launch with this tree has a cooperative kernel, and gives it no rays
+    nine = C.Scene("\n".join(S.balanced("Union", [S.sphere((30 + i, 0, 0), "5AC85A", 0.2) for i in range(9)])) + "\n")
+    cam, light, phong = C.camera_look_at((2.2, 1.3, 2.9), (0, 0, 0), 45), C.light(LIGHT), C.phong(*PHONG)
+    ref = small.render(cam, light, phong, 48, 48, coop=-1)
+    far = nine.render(cam, light, phong, 8, 8, coop=-1)
+    out, rest = C.alloc_outputs(48, 48), [C.alloc_outputs(8, 8) for _ in range(1024)]
+
+    def clear():
+        for o in [out] + rest:
+            for t in o.values():
+                t.fill_(77)
+
+    # in one launch the small tree's rays do go to the cooperative kernel
+    clear()
+    before = C.coop_rays()
+    C.render_batch(C.make_jobs([(small, cam, light, phong, 48, 48, out), (nine, cam, light, phong, 8, 8, rest[0])]))
+    assert C.coop_rays() > before
+    for key in KEYS:
+        assert torch.equal(out[key].view(torch.uint8), ref[key].view(torch.uint8)), key
+    # in the second of two launches, the first of which has a cooperative kernel, they end in their lanes
+    clear()
+    before = C.coop_rays()
+    print("[case] 1024 + 1 jobs", flush=True)
+    C.render_batch(C.make_jobs([(nine, cam, light, phong, 8, 8, o) for o in rest] +
+                               [(small, cam, light, phong, 48, 48, out)]))
+    assert C.coop_rays() == before
+    for key in KEYS:
+        assert torch.equal(out[key].view(torch.uint8), ref[key].view(torch.uint8)), key
+        for o in rest:
+            assert torch.equal(o[key].view(torch.uint8), far[key].view(torch.uint8)), key
+    # and the stream's next hand-over finds an empty list
+    clear()
+    C.render_batch(C.make_jobs([(small, cam, light, phong, 48, 48, out), (nine, cam, light, phong, 8, 8, rest[0])]))
+    torch.cuda.synchronize()
+    for key in KEYS:
+        assert torch.equal(out[key].view(torch.uint8), ref[key].view(torch.uint8)), key
+    small.close()
+    nine.close()
