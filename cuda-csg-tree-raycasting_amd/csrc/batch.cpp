@@ -186,18 +186,15 @@ csg_status Stage(csg_batch* b) {
     const int32_t cnt = c < static_cast<int32_t>(plan.chunks.size()) ? plan.chunks[c].second : 0;
     if (cnt > ch.cap) return Fail(CSG_E_ARG, "csg_batch: chunk capacity exceeded");
     int64_t base = 0;
-    int32_t depth = 1, maxOps = 1, maxLeaves = 1;
-    bool anyInBoxes = false, anyGroups = false;
+    int32_t depth = 1;
+    LaunchScenes scenes(1);
     for (int32_t i = 0; i < cnt; i++) {
       const csg_job& j = b->jobs[plan.order[start + i]];
-      maxOps = std::max(maxOps, j.scene->dev.nOps);
-      maxLeaves = std::max(maxLeaves, j.scene->dev.opLeaves);
-      anyInBoxes |= j.scene->dev.conservative != 0;
-      anyGroups |= HasTileGroups(j.scene);
       const csg_status st = BuildJob(j.scene, &j.camera, &j.light, &j.phong, j.width, j.height, &j.out, &b->opts,
                                      b->device, base, &ch.hostJobs[i]);
       if (st != CSG_OK) return st;
       base += ch.hostJobs[i].tiles;
+      scenes.Add(j.scene, ch.hostJobs[i].tiles, b->cfg.mode);
       depth = std::max(depth, j.scene->dev.opDepth);
     }
     csgray::RenderParams& p = ch.params;
@@ -213,7 +210,7 @@ csg_status Stage(csg_batch* b) {
     if (e != hipSuccess) return FailHip(e, "choosing the launch shape");
     csgray::FitGridToTiles(&ch.shape, base);
     p.totalWaves = static_cast<uint32_t>(ch.shape.grid) * static_cast<uint32_t>(ch.shape.block / 64);
-    PrepareCoop(b->cfg, maxOps, maxLeaves, anyInBoxes, anyGroups, ch.heavy, ch.shape, &p);
+    PrepareCoop(b->cfg, scenes, ch.heavy, ch.shape, &p);
   }
   return CSG_OK;
 }

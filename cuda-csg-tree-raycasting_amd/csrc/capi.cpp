@@ -190,29 +190,88 @@ int32_t DefaultCoopGraceMille(int64_t waves, int64_t tiles, bool batched, bool l
   return static_cast<int32_t>(std::min<int64_t>(std::max<int64_t>(g, 5), batched ? 1000000 : 3000));
 }
 
-void PrepareCoop(const LaunchConfig& cfg, int32_t maxOps, int32_t maxLeaves, bool anyInBoxes, bool anyGroups,
-                 uint2* heavy, const LaunchShape& shape, RenderParams* p) {
+// Unions of flush parts (scene.hpp, flushParts).  A tie of two members fails a
+// ray in a group, while the walk operator by operator follows most ties to
+// their end: no groups for small trees of which a quarter is flush, and for
+// any from kTiesTiles tiles on where flush parts x tiles reach kTiesWork x
+// parts.  On a grid, with the group and without: 24 cubes 320x184 68 and 43 us,
+// 640x360 101 and 46, 1920x1080 447 and 174; 64 cubes 320x184 139 and 157,
+// 640x360 291 and 172; 200 cubes 480x272 553 and 598, 640x360 776 and 653; 64
+// cylinders (10 of them flush) 640x360 107 and 137, 960x544 143 and 148,
+// 1280x720 201 and 175.
+constexpr int32_t kFlushShare = 4, kFlushSmallOps = 48;
+constexpr int64_t kTiesTiles = 3000, kTiesWork = 750;
+// The rays that fail all the same take a wave each in the next kernel, which
+// costs a large frame more than whole tiles save.  Per lane and by tiles: 24
+// cubes 1280x720 81 and 83 us; 64 cubes 640x360 209 and 172, 1280x720 182 and
+// 252; 200 cubes 640x360 601 and 653, 960x544 671 and 1153; 200 with a piece cut
+// from each 640x360 718 and 476, 960x544 1082 and 728, 1920x1080 1043 and 1988;
+// 500 cubes 480x272 1135 and 1041, 640x360 1274 and 1417.  In exact mode 500
+// cubes 640x360 1416 and 1974, 1920x1080 4738 and 9233, but 200 cylinders
+// 960x544 1389 and 763, 200 mixed parts 960x544 1415 and 1061, 1920x1080 2050
+// and 2571.
+constexpr int32_t kFlushLargeOps = 400;
+constexpr int64_t kFlushTiles = 6144;
+constexpr double kFlushTileUs = 0.1;  // about what a tile loses
+// What the other jobs of a batch lose by the per-lane kernel: trees below
+// kLaneLargeOps operators 0.5 ns a tile and operator (16 frames of the
+// Wikipedia scene at 512x512: 117 us by tiles, 240 per lane), larger ones 0.25
+// ns, 0.7 in exact mode, and no less than a millisecond, the longest rays'
+// time whatever the frame's size (24 random trees 128x128 to 512x512: 399 and
+// 2406 us, exact mode 1102 and 6570).
+constexpr int32_t kLaneLargeOps = 64;
+constexpr double kLaneSmallUs = 0.0005, kLaneLargeUs = 0.00025, kLaneLargeExactUs = 0.0007, kLaneLeastUs = 1000;
+
+void LaunchScenes::Add(const csg_scene* s, int64_t tiles, Mode mode) {
+  const int32_t ops = s->dev.nOps;
+  maxOps = std::max(maxOps, ops);
+  maxLeaves = std::max(maxLeaves, s->dev.opLeaves);
+  inBoxes |= s->dev.conservative != 0;
+  const int64_t flush = s->flat.flushParts, parts = s->flat.nPrims;
+  const bool quarter = flush > 0 && kFlushShare * flush >= parts;
+  const bool ties = (quarter && ops < kFlushSmallOps) || (tiles >= kTiesTiles && flush * tiles >= kTiesWork * parts);
+  groups |= HasTileGroups(s) && !ties;
+  if (quarter && (ops >= kFlushLargeOps ? tiles >= kTiesTiles
+                                        : mode == Mode::kFast && ops >= kFlushSmallOps && tiles >= kFlushTiles))
+    byTiles += kFlushTileUs * static_cast<double>(tiles);
+  else if (ops >= kLaneLargeOps)
+    largeWork += tiles * ops;
+  else
+    byLanes += kLaneSmallUs * static_cast<double>(tiles * ops);
+}
+
+bool LaunchScenes::KeepsLanes(Mode mode) const {
+  double lost = byLanes;
+  if (largeWork > 0)
+    lost += std::max(kLaneLeastUs,
+                     (mode == Mode::kFast ? kLaneLargeUs : kLaneLargeExactUs) * static_cast<double>(largeWork));
+  return byTiles > lost;
+}
+
+void PrepareCoop(const LaunchConfig& cfg, const LaunchScenes& scenes, uint2* heavy, const LaunchShape& shape,
+                 RenderParams* p) {
   // (a launch without a cooperative kernel must not hand rays over, whatever
   // an earlier launch left in `p`)
   p->budget = 0;
   p->heavy = nullptr;
   p->heavyCap = 0;
   p->coopWaves = 0;
-  PlanTiles(cfg, anyGroups, anyInBoxes, maxOps, p);
+  p->tileSlots = 0;
+  if (!scenes.KeepsLanes(cfg.mode)) PlanTiles(cfg, scenes.groups, scenes.inBoxes, scenes.maxOps, p);
   if (!heavy) return;
   // Trees whose crossings always fit the tile kernel's lists, two a primitive,
   // leave a few rays in millions (ties), which a lane finishes in at most a
   // microsecond an operator; a cooperative launch, found empty, takes 4 us.
-  if (p->tileSlots > 0 && 2 * (maxOps + 1) <= kTilePlainSlots) return;
-  const bool lists = CoopLists(cfg, anyInBoxes);
-  const CoopPlan c = PlanCoop(cfg, maxOps, maxLeaves, lists);
+  if (p->tileSlots > 0 && 2 * (scenes.maxOps + 1) <= kTilePlainSlots) return;
+  const bool lists = CoopLists(cfg, scenes.inBoxes);
+  const CoopPlan c = PlanCoop(cfg, scenes.maxOps, scenes.maxLeaves, lists);
   if (c.budget <= 0) return;
   p->budget = c.budget;
   p->heavy = heavy;
   p->heavyCap = kHeavyCap;
   p->resume = reinterpret_cast<uint32_t*>(heavy + kHeavyCap);
   p->resumeBytes = static_cast<uint32_t>(kResumeBytes);
-  p->coopOps = maxOps;
+  p->coopOps = scenes.maxOps;
   p->coopLists = lists ? 1 : 0;
   p->coopQueueCap = c.queueCap;
   p->coopWaves = c.waves;
@@ -709,7 +768,9 @@ csg_status csg_render_ex(const csg_scene* s, const csg_camera* cam, const csg_li
     if (hsd != CSG_OK) return hsd;
   }
   cfg.tiles = cfg.tiles && cfg.sceneInLds == -1 && !p.tileOrder;
-  PrepareCoop(cfg, s->dev.nOps, s->dev.opLeaves, s->dev.conservative != 0, HasTileGroups(s), heavy, shape, &p);
+  LaunchScenes scenes(0);
+  scenes.Add(s, p.numTiles, cfg.mode);
+  PrepareCoop(cfg, scenes, heavy, shape, &p);
   e = csgray::LaunchRender(p, cfg, shape, hs);
   if (e != hipSuccess) return FailHip(e, "render launch");
   return CSG_OK;
@@ -778,15 +839,9 @@ csg_status csg_render_batch(const csg_job* jobs, int32_t njobs, const csg_render
       const csg_status hsd = HeavyFor(dev, hs, &heavy);
       if (hsd != CSG_OK) return hsd;
     }
-    int32_t maxOps = 1, maxLeaves = 1;
-    bool anyInBoxes = false, anyGroups = false;
-    for (int32_t i = 0; i < n; i++) {
-      maxOps = std::max(maxOps, jobs[start + i].scene->dev.nOps);
-      maxLeaves = std::max(maxLeaves, jobs[start + i].scene->dev.opLeaves);
-      anyInBoxes |= jobs[start + i].scene->dev.conservative != 0;
-      anyGroups |= HasTileGroups(jobs[start + i].scene);
-    }
-    PrepareCoop(cfg, maxOps, maxLeaves, anyInBoxes, anyGroups, heavy, shape, &p);
+    LaunchScenes scenes(1);
+    for (int32_t i = 0; i < n; i++) scenes.Add(jobs[start + i].scene, host[i].tiles, cfg.mode);
+    PrepareCoop(cfg, scenes, heavy, shape, &p);
     e = csgray::LaunchRender(p, cfg, shape, hs);
     if (e != hipSuccess) return FailHip(e, "batched render launch");
   }

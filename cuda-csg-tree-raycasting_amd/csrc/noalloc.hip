@@ -115,8 +115,9 @@ extern "C" csg_status csg_render_noalloc(const csg_scene* s, const csg_camera* c
   p.queue = reinterpret_cast<uint32_t*>(base);
   uint2* heavy = reinterpret_cast<uint2*>(base + kQueueRegion);
   cfg.tiles = cfg.tiles && cfg.sceneInLds == -1 && !p.tileOrder;
-  PrepareCoop(cfg, s->dev.nOps, s->dev.opLeaves, s->dev.conservative != 0, HasTileGroups(s),
-              cfg.budget >= 0 ? heavy : nullptr, shape, &p);
+  LaunchScenes scenes(0);
+  scenes.Add(s, p.numTiles, cfg.mode);
+  PrepareCoop(cfg, scenes, cfg.budget >= 0 ? heavy : nullptr, shape, &p);
   p.resumeBytes = static_cast<uint32_t>(kNoAllocResumeBytes);
   e = csgray::LaunchRender(p, cfg, shape, hs);
   if (e != hipSuccess) return FailHip(e, "render launch");

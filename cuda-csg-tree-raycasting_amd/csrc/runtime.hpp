@@ -33,6 +33,20 @@ size_t SceneBytes(const csg_scene* s);
 // Whether the tile kernel takes Union groups of the scene.
 inline bool HasTileGroups(const csg_scene* s) { return s->dev.tileOps != s->dev.ivOps; }
 
+// The scenes of one launch, as the choice of its kernels needs them.
+struct LaunchScenes {
+  int32_t maxOps, maxLeaves;
+  bool inBoxes = false, groups = false;
+  // what the launch would lose by whole tiles, and what without them (us)
+  double byTiles = 0, byLanes = 0;
+  int64_t largeWork = 0;  // tiles x operators of trees of kLaneLargeOps operators and more
+  explicit LaunchScenes(int32_t least) : maxOps(least), maxLeaves(least) {}
+  // A job of `tiles` 8x8 tiles (all samples).
+  void Add(const csg_scene* s, int64_t tiles, Mode mode);
+  // Whether the launch keeps the per-lane kernel, whatever its options.
+  bool KeepsLanes(Mode mode) const;
+};
+
 // Validates one job and fills its device descriptor; `tileBase` is its first
 // queue index within the launch.
 csg_status BuildJob(const csg_scene* s, const csg_camera* cam, const csg_light* light, const csg_phong* phong,
@@ -45,11 +59,11 @@ csg_status QueueFor(int dev, hipStream_t stream, uint32_t** out);
 // The heavy-ray list of (device, stream).
 csg_status HeavyFor(int dev, hipStream_t stream, uint2** out);
 
-// Fills the cooperative-evaluation fields of `p` for a launch whose scenes
-// have at most `maxOps` operators (deferral off when the options say so or
-// the cooperative kernel's state does not fit LDS).
-void PrepareCoop(const LaunchConfig& cfg, int32_t maxOps, int32_t maxLeaves, bool anyInBoxes, bool anyGroups,
-                 uint2* heavy, const LaunchShape& shape, RenderParams* p);
+// Fills the tile kernel's and the cooperative kernel's fields of `p`
+// (deferral off when the options say so or the cooperative kernel's state
+// does not fit LDS).
+void PrepareCoop(const LaunchConfig& cfg, const LaunchScenes& scenes, uint2* heavy, const LaunchShape& shape,
+                 RenderParams* p);
 
 // Copies a job table to the (device, stream) table buffer in stream order.
 csg_status UploadJobs(int dev, hipStream_t stream, const Job* jobs, size_t n, const Job** out);

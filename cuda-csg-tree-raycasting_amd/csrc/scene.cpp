@@ -6,6 +6,7 @@
 #include <cmath>
 #include <cstring>
 #include <string_view>
+#include <tuple>
 
 namespace csgray {
 
@@ -128,6 +129,60 @@ bool CylinderInBox(const Primitive& p) {
     if (ext > e * (1.0 + 1e-6)) return false;
   }
   return true;
+}
+
+// An axis-aligned face: its plane and its extent along the other two axes.
+struct Face {
+  int32_t side;  // 2 x axis + (0 low, 1 high)
+  float at, lo[2], hi[2];
+  int32_t member, prim;
+};
+
+// Adds the faces of primitive `q`: a cube's six, the caps of a cylinder whose
+// axis is a coordinate axis.
+void AddFaces(const Primitive& q, int32_t member, int32_t prim, std::vector<Face>* out) {
+  if (q.type == kSphere) return;
+  const float c[3] = {q.x, q.y, q.z};
+  int along = -1;  // a cylinder's axis
+  if (q.type == kCylinder) {
+    for (int k = 0; k < 3; k++)
+      if (std::fabs(std::fabs(q.axis[k]) - 1.0f) < 1e-6f) along = k;
+    if (along < 0) return;
+  }
+  float lo[3], hi[3];
+  for (int k = 0; k < 3; k++) {
+    const float e = q.type == kCube ? q.size / 2 : (k == along ? q.height / 2 : q.radius);
+    lo[k] = c[k] - e;
+    hi[k] = c[k] + e;
+    if (!std::isfinite(lo[k]) || !std::isfinite(hi[k])) return;
+  }
+  for (int k = 0; k < 3; k++) {
+    if (along >= 0 && k != along) continue;
+    const int a = (k + 1) % 3, b = (k + 2) % 3;
+    out->push_back(Face{2 * k, lo[k], {lo[a], lo[b]}, {hi[a], hi[b]}, member, prim});
+    out->push_back(Face{2 * k + 1, hi[k], {lo[a], lo[b]}, {hi[a], hi[b]}, member, prim});
+  }
+}
+
+// How many primitives have a face in one plane with, facing the same way as
+// and overlapping a face of another member: rays through both cross them at
+// one time (a tie).  Each face is compared with the next kNear of its plane.
+int32_t CountFlush(std::vector<Face>& faces, size_t prims) {
+  constexpr size_t kNear = 64;
+  std::sort(faces.begin(), faces.end(), [](const Face& x, const Face& y) {
+    return std::tie(x.side, x.at, x.lo[0]) < std::tie(y.side, y.at, y.lo[0]);
+  });
+  std::vector<uint8_t> flush(prims, 0);
+  for (size_t i = 0; i < faces.size(); i++) {
+    const Face& x = faces[i];
+    for (size_t j = i + 1; j < std::min(faces.size(), i + 1 + kNear); j++) {
+      const Face& y = faces[j];
+      if (y.side != x.side || y.at != x.at || !(y.lo[0] < x.hi[0])) break;
+      if (x.member != y.member && x.lo[1] < y.hi[1] && y.lo[1] < x.hi[1])
+        flush[static_cast<size_t>(x.prim)] = flush[static_cast<size_t>(y.prim)] = 1;
+    }
+  }
+  return static_cast<int32_t>(std::count(flush.begin(), flush.end(), uint8_t{1}));
 }
 
 }  // namespace
@@ -384,6 +439,7 @@ FlatScene Flatten(const CSGTree& tree) {
     f.walkOps = f.ivOps;
     std::vector<int32_t> members, todo;
     std::vector<int32_t> roots;
+    std::vector<Face> faces;
     for (int32_t i = 0; i < f.nNodes; i++) {
       const CSGNode& n = tree.nodes[i];
       if (n.primitiveIdx == -1 && n.type == kUnion && (n.parent < 0 || tree.nodes[n.parent].type != kUnion))
@@ -481,14 +537,31 @@ FlatScene Flatten(const CSGTree& tree) {
         if (f.tileOps.empty()) f.tileOps = f.ivOps;
         f.tileOps[4 * static_cast<size_t>(gi) + 3] = w;
         inTileGroups += members.size();
+        // the faces of what the members consist of, without what is cut from it
+        faces.clear();
+        for (const int32_t m : members) {
+          todo.assign(1, m);
+          while (!todo.empty()) {
+            const CSGNode& n = tree.nodes[todo.back()];
+            todo.pop_back();
+            if (n.primitiveIdx != -1) {
+              AddFaces(tree.primitives[n.primitiveIdx], m, n.primitiveIdx, &faces);
+            } else {
+              todo.push_back(n.left);
+              if (n.type != kDifference) todo.push_back(n.right);
+            }
+          }
+        }
+        f.flushParts += CountFlush(faces, tree.primitives.size());
       }
       f.unionGroups++;
     }
   }
-  // Groups that hold few of a scene's primitives are not worth the kernel that
-  // walks them, which runs half as many waves and goes over a ray whose list
-  // overflows in stretches: mixed trees of 796 at 624x624 take 5.6 ms with it,
-  // 1.8 ms without, of 900 at 1280x720 4.9 and 2.8 ms.
+  // Groups of few members beside a scene's primitives are not worth the kernel
+  // that walks them, which runs half as many waves and goes over a ray whose
+  // list overflows in stretches: mixed trees of 796 at 624x624 take 5.6 ms with
+  // it, 1.8 ms without, of 900 at 1280x720 4.9 and 2.8 ms.  (Members are
+  // counted, not what they consist of.)
   if (4 * inTileGroups < static_cast<size_t>(f.nPrims)) f.tileOps.clear();
   return f;
 }

@@ -179,8 +179,8 @@ void Dispatch(csg_server* s, Slot& sl) {
   std::vector<int64_t> run;
   jobs.reserve(take.size());
   int64_t base = 0;
-  int32_t depth = 1, maxOps = 1, maxLeaves = 1;
-  bool anyInBoxes = false, anyGroups = false;
+  int32_t depth = 1;
+  LaunchScenes scenes(1);
   csg_render_opts opts{};
   opts.mode = s->cfg.mode;
   bool failed = false;
@@ -212,10 +212,7 @@ void Dispatch(csg_server* s, Slot& sl) {
     run.push_back(tk);
     base += jb.tiles;
     depth = std::max(depth, sc->dev.opDepth);
-    maxOps = std::max(maxOps, sc->dev.nOps);
-    maxLeaves = std::max(maxLeaves, sc->dev.opLeaves);
-    anyInBoxes |= sc->dev.conservative != 0;
-    anyGroups |= HasTileGroups(sc);
+    scenes.Add(sc, jb.tiles, s->launch.mode);
     r.state = kRunning;
   }
   if (failed) s->doneCv.notify_all();
@@ -238,7 +235,7 @@ void Dispatch(csg_server* s, Slot& sl) {
     p.queue = queue;
     csgray::FitGridToTiles(&shape, base);
     p.totalWaves = static_cast<uint32_t>(shape.grid) * static_cast<uint32_t>(shape.block / 64);
-    PrepareCoop(s->launch, maxOps, maxLeaves, anyInBoxes, anyGroups, heavy, shape, &p);
+    PrepareCoop(s->launch, scenes, heavy, shape, &p);
     if (csgray::LaunchRender(p, s->launch, shape, sl.stream) != hipSuccess) st = CSG_E_HIP;
   }
   if (st == CSG_OK && hipEventRecord(sl.done, sl.stream) != hipSuccess) st = CSG_E_HIP;

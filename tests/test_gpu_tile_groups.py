@@ -125,3 +125,53 @@ def test_the_first_crossing_before_a_flush_cut(gpu):
     assert int(out["prim_id"][16, 16]) == 0
     assert abs(float(out["depth"][16, 16]) - 3.5) < 0.01
     scene.close()
+
+
+def _flush_cubes(n, seed, cut=False):
+    """A Union of n cubes on a grid, many with faces in one plane; `cut`: each with a flush piece cut off."""
+    rng = np.random.default_rng(seed)
+    leaves = []
+    for _ in range(n):
+        c = list(_grid(rng, 0.25))
+        leaf = S.cube(c, "C85A5A", 0.5 if cut else float(rng.integers(1, 5)) * 0.25)
+        if cut:
+            c[int(rng.integers(0, 3))] += 0.25
+            leaf = "\n".join(["Difference", leaf, S.cube(c, "5A5AC8", 0.5)])
+        leaves.append(leaf)
+    return "\n".join(S.balanced("Union", leaves)) + "\n"
+
+
+# Unions of flush parts: too few members for a group, a group of few, groups kept up to 3000 tiles
+# (432x432 has 2916, 440x440 3025), and by the per-lane kernel: in fast mode from 48 operators
+# and 6144 tiles on (624x624 has 6084, 632x632 6241), from 400 operators and 3000 tiles in both modes
+@pytest.mark.parametrize("mode", [C.MODE_FAST, C.MODE_EXACT], ids=["fast", "exact"])
+@pytest.mark.parametrize("n,cut", [(23, False), (24, False), (24, True), (48, False), (49, False), (200, True), (400, False), (401, False)])
+def test_flush_unions_equal_the_state_machine(gpu, n, cut, mode):
+    scene = C.Scene(_flush_cubes(n, n, cut))
+    specs, refs = [], []
+    for size, view in zip([97, 432, 440, 624, 632], VIEWS + VIEWS[:2]):
+        print(f"[case] {n} cubes, cut {cut}, {size}x{size}", flush=True)
+        got = _frame(scene, view, size, size, mode=mode)
+        ref = _frame(scene, view, size, size, mode=mode, coop=-1)
+        _same(got, ref, size)
+        eye, target, fov = view
+        specs.append((scene, C.camera_look_at(eye, target, fov), C.light(LIGHT), C.phong(*PHONG), size, size,
+                      C.alloc_outputs(size, size)))
+        refs.append(ref)
+    small = C.Scene(S.WIKIPEDIA)
+    eye, target, fov = VIEWS[1]
+    specs.append((small, C.camera_look_at(eye, target, fov), C.light(LIGHT), C.phong(*PHONG), 300, 200,
+                  C.alloc_outputs(300, 200)))
+    refs.append(_frame(small, VIEWS[1], 300, 200, mode=mode, coop=-1))
+    C.render_batch(C.make_jobs(specs), mode=mode)
+    batch = C.Batch(C.make_jobs(specs), mode=mode)
+    for spec, ref in zip(specs, refs):
+        _same(spec[6], ref, "batch")
+        for t in spec[6].values():
+            t.fill_(0)
+    batch.launch()
+    for spec, ref in zip(specs, refs):
+        _same(spec[6], ref, "captured batch")
+    batch.close()
+    scene.close()
+    small.close()
