@@ -213,6 +213,22 @@ constexpr int64_t kTiesTiles = 3000, kTiesWork = 750;
 constexpr int32_t kFlushLargeOps = 400;
 constexpr int64_t kFlushTiles = 6144;
 constexpr double kFlushTileUs = 0.1;  // about what a tile loses
+// A large tree with groups in few tiles, under a third of its operators: each
+// tile sees much of the scene, and its walk, one chain, outlasts the rays' time
+// per lane by about kFewChainUs an operator (less in more tiles, more in the
+// largest trees; in exact mode kFewChainExactUs an operator beyond
+// kFewExactOps).  Such jobs lose kFew*Us a tile and operator per lane, where
+// the cooperative kernel merges intervals little of it.  Beside 16 frames of the
+// Wikipedia scene at 512x512, per lane and by tiles: 500 spheres taken from a
+// cube at 64x64 313 and 393 us, 1000 332 and 618, at 128x128 369 and 481, 1500
+// at 64x64 351 and 822; 1500 spheres and cylinders 604 and 1138, exact mode 1315
+// and 2785.  40 such jobs alone: 1000 spheres 64x64 333 and 622 us, 16 at
+// 128x128 648 and 468; 1000 spheres and cylinders 64x64 1090 and 831; 4000 11.5
+// and 18.0 ms.  (One tree of 4000 alone, 192x192 3.9 and 6.1 ms, 256x256 5.8 and 5.0.)
+constexpr int64_t kFewTiles = 768;
+constexpr double kFewChainUs = 0.4, kFewChainExactUs = 1.5;
+constexpr int32_t kFewExactOps = 500, kFewLargestOps = 2048;
+constexpr double kFewInBoxesUs = 0.00008, kFewUs = 0.0004, kFewExactUs = 0.00025;
 // What the other jobs of a batch lose by the per-lane kernel: trees below
 // kLaneLargeOps operators 0.5 ns a tile and operator (16 frames of the
 // Wikipedia scene at 512x512: 117 us by tiles, 240 per lane), larger ones 0.25
@@ -232,12 +248,19 @@ void LaunchScenes::Add(const csg_scene* s, int64_t tiles, Mode mode) {
   const bool ties = (quarter && ops < kFlushSmallOps) || (tiles >= kTiesTiles && flush * tiles >= kTiesWork * parts);
   groups |= HasTileGroups(s) && !ties;
   if (quarter && (ops >= kFlushLargeOps ? tiles >= kTiesTiles
-                                        : mode == Mode::kFast && ops >= kFlushSmallOps && tiles >= kFlushTiles))
+                                        : mode == Mode::kFast && ops >= kFlushSmallOps && tiles >= kFlushTiles)) {
     byTiles += kFlushTileUs * static_cast<double>(tiles);
-  else if (ops >= kLaneLargeOps)
+  } else if (HasTileGroups(s) && ops >= kTileLargeOps && tiles < kFewTiles && 3 * tiles < ops) {
+    const bool fast = mode == Mode::kFast;
+    const double walk = fast ? kFewChainUs * ops * (ops > kFewLargestOps ? 3 : 1)
+                             : kFewChainExactUs * std::max(0, ops - kFewExactOps);
+    chain = std::max(chain, walk * (1 - 1.5 * static_cast<double>(tiles) / ops));
+    byLanes += (!fast ? kFewExactUs : s->dev.conservative ? kFewInBoxesUs : kFewUs) * static_cast<double>(tiles * ops);
+  } else if (ops >= kLaneLargeOps) {
     largeWork += tiles * ops;
-  else
+  } else {
     byLanes += kLaneSmallUs * static_cast<double>(tiles * ops);
+  }
 }
 
 bool LaunchScenes::KeepsLanes(Mode mode) const {
@@ -245,7 +268,7 @@ bool LaunchScenes::KeepsLanes(Mode mode) const {
   if (largeWork > 0)
     lost += std::max(kLaneLeastUs,
                      (mode == Mode::kFast ? kLaneLargeUs : kLaneLargeExactUs) * static_cast<double>(largeWork));
-  return byTiles > lost;
+  return byTiles + chain > lost;
 }
 
 void PrepareCoop(const LaunchConfig& cfg, const LaunchScenes& scenes, uint2* heavy, const LaunchShape& shape,

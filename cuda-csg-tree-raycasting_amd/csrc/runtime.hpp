@@ -39,6 +39,7 @@ struct LaunchScenes {
   bool inBoxes = false, groups = false;
   // what the launch would lose by whole tiles, and what without them (us)
   double byTiles = 0, byLanes = 0;
+  double chain = 0;       // of byTiles: the longest walk of a large tree in few tiles, beyond its time per lane
   int64_t largeWork = 0;  // tiles x operators of trees of kLaneLargeOps operators and more
   explicit LaunchScenes(int32_t least) : maxOps(least), maxLeaves(least) {}
   // A job of `tiles` 8x8 tiles (all samples).

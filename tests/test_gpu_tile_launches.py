@@ -61,3 +61,35 @@ def test_a_later_launch_of_small_trees_finishes_its_rays(gpu):
         assert torch.equal(out[key].view(torch.uint8), ref[key].view(torch.uint8)), key
     small.close()
     nine.close()
+
+
+# A launch keeps the per-lane kernel for large trees with groups in few tiles (64x64: 64 tiles; 1000
+# spheres to 327 tiles, 144x144 324 and 152x152 361) unless its other jobs, small trees or large ones, outweigh them
+@pytest.mark.parametrize("mode", [C.MODE_FAST, C.MODE_EXACT], ids=["fast", "exact"])
+@pytest.mark.parametrize("others", ["none", "small", "large"])
+@pytest.mark.parametrize("n,size", [(447, 64), (448, 64), (1000, 144), (1000, 152)])
+def test_large_trees_in_few_tiles(gpu, n, size, others, mode):
+    light, phong = C.light(LIGHT), C.phong(*PHONG)
+    cam = C.camera_look_at((2.2, 1.3, 2.9), (0, 0, 0), 55)
+    big, wiki = C.Scene(S.cheese(n, seed=n)), C.Scene(S.WIKIPEDIA)
+    mixed = C.Scene("\n".join(S.random_ops_balanced(np.random.default_rng(3), [
+        S.cube(tuple(np.random.default_rng(i).uniform(-1, 1, 3)), "3CC850", 0.8) for i in range(80)])) + "\n")
+    scenes = {"none": [(big, size)] * 34, "small": [(big, size)] + [(wiki, 400)] * 3,
+              "large": [(big, size)] + [(mixed, 400)] * 3}[others]
+    specs = [(sc, cam, light, phong, s, s, C.alloc_outputs(s, s)) for sc, s in scenes]
+    refs = {sc: sc.render(cam, light, phong, s, s, mode=mode, coop=-1) for sc, s in scenes}
+    jobs = C.make_jobs(specs)
+    print(f"[case] {n} spheres {size}x{size}, others {others}", flush=True)
+    batch = C.Batch(jobs, mode=mode)
+    for launch in (lambda: C.render_batch(jobs, mode=mode), batch.launch):
+        for spec in specs:
+            for t in spec[6].values():
+                t.fill_(77)
+        launch()
+        torch.cuda.synchronize()
+        for spec in specs:
+            for key in KEYS:
+                assert torch.equal(spec[6][key].view(torch.uint8), refs[spec[0]][key].view(torch.uint8)), key
+    batch.close()
+    for sc in (big, wiki, mixed):
+        sc.close()
