@@ -187,14 +187,15 @@ def bench_batched(torch, C, S, reps, coop):
     batch_ms = _time_ms(torch, lambda: C.render_batch(jobs, **coop), reps)
     batch = C.Batch(jobs, **coop)
     tune = batch.autotune(reps=2)
+    whole_tiles = batch.whole_tiles()
     graph_ms = _time_ms(torch, batch.launch, reps)
     batch.close()
     return {"workload": "256 random trees (2-1024 leaves, balanced, ops uniform), 128^2..1024^2, orbit cameras",
             "rays": rays, "plain_per_scene_mrays_s": round(rays / plain_ms / 1e3, 1),
             "batched_mrays_s": round(rays / batch_ms / 1e3, 1), "graph_mrays_s": round(rays / graph_ms / 1e3, 1),
             "batched_vs_plain": round(plain_ms / min(batch_ms, graph_ms), 2),
-            "autotune": {"block": tune.block, "tile_walk": tune.tile_walk, "heaviest_first": tune.heaviest_first,
-                         "depth_split": tune.depth_split},
+            "autotune": {"whole_tiles": whole_tiles, "block": tune.block, "tile_walk": tune.tile_walk,
+                         "heaviest_first": tune.heaviest_first, "depth_split": tune.depth_split},
             "ms": {"plain": round(plain_ms, 2), "batched": round(batch_ms, 2), "graph": round(graph_ms, 2)}}
 
 
@@ -233,6 +234,7 @@ def bench_stress(torch, C, S, reps, coop):
     jobs = C.make_jobs([(scene, cam, light, ph, w, h, bouts)])
     batch = C.Batch(jobs, samples=spp, seed=seed, **coop)
     tune = batch.autotune(reps=1)
+    whole_tiles = batch.whole_tiles()
     graph_ms = _time_ms(torch, batch.launch, reps)
     same = all(np.array_equal(plain_img[k].view(np.uint8), bouts[k].cpu().numpy().view(np.uint8))
                for k in ("rgba", "depth", "prim_id", "flags"))
@@ -246,8 +248,8 @@ def bench_stress(torch, C, S, reps, coop):
             "rays": rays, "nodes": info.nodes, "op_depth": info.op_depth, "scene_in_lds": bool(plan.scene_in_lds),
             "plain_ms": round(plain_ms, 2), "plain_mrays_s": round(rays / plain_ms / 1e3, 1),
             "graph_ms": round(graph_ms, 2), "graph_mrays_s": round(rays / graph_ms / 1e3, 1),
-            "autotune": {"block": tune.block, "tile_walk": tune.tile_walk, "heaviest_first": tune.heaviest_first,
-                         "depth_split": tune.depth_split},
+            "autotune": {"whole_tiles": whole_tiles, "block": tune.block, "tile_walk": tune.tile_walk,
+                         "heaviest_first": tune.heaviest_first, "depth_split": tune.depth_split},
             "coop_rays_per_frame": round(handed), "plain_equals_batched": same, "_gpu_rows64": rows64}
 
 

@@ -153,6 +153,7 @@ _SIGNATURES = [
     ("csg_batch_update", ctypes.c_int, [_P, ctypes.c_void_p, ctypes.c_int32, _P]),
     ("csg_batch_launch", ctypes.c_int, [_P, _P]),
     ("csg_batch_autotune", ctypes.c_int, [_P, ctypes.c_int32, _P, ctypes.POINTER(BatchTuning)]),
+    ("csg_batch_whole_tiles", ctypes.c_int, [_P, ctypes.POINTER(ctypes.c_int32)]),
     ("csg_batch_free", ctypes.c_int, [_P]),
     ("csg_server_create", ctypes.c_int, [ctypes.POINTER(ServerConfig), ctypes.POINTER(_P)]),
     ("csg_server_add_scene", ctypes.c_int, [_P, _P, ctypes.POINTER(ctypes.c_int32)]),
@@ -465,9 +466,16 @@ class Batch:
         self.jobs = jobs
 
     def autotune(self, reps=2, stream=None) -> BatchTuning:
+        """Keeps the fastest launch shape; `block` of the result is the one to pass on unless whole_tiles()."""
         t = BatchTuning()
         _check(lib().csg_batch_autotune(self.handle, int(reps), self._stream(stream), ctypes.byref(t)))
         return t
+
+    def whole_tiles(self) -> bool:
+        """Whether launches of the batch classify whole tiles (block=0 gives that choice again)."""
+        v = ctypes.c_int32()
+        _check(lib().csg_batch_whole_tiles(self.handle, ctypes.byref(v)))
+        return bool(v.value)
 
     def close(self):
         if getattr(self, "handle", None):

@@ -501,6 +501,14 @@ csg_status csg_batch_autotune(csg_batch* b, int32_t reps, void* stream, csg_batc
   return CSG_OK;
 }
 
+csg_status csg_batch_whole_tiles(const csg_batch* b, int32_t* whole_tiles) {
+  if (!b || !whole_tiles) return Fail(CSG_E_ARG, "csg_batch_whole_tiles: NULL argument");
+  *whole_tiles = std::any_of(b->chunks.begin(), b->chunks.end(), [](const Chunk& c) {
+                   return c.params.tileSlots > 0 && c.params.numTiles > 0;
+                 }) ? 1 : 0;
+  return CSG_OK;
+}
+
 csg_status csg_batch_free(csg_batch* b) {
   if (!b) return CSG_OK;
   if (b->staged) {

@@ -274,22 +274,25 @@ csg_status csg_batch_create(const csg_job* jobs, int32_t njobs, const csg_render
  * the graph's kernel nodes get new parameters. */
 csg_status csg_batch_update(csg_batch* batch, const csg_job* jobs, int32_t njobs, void* stream);
 csg_status csg_batch_launch(csg_batch* batch, void* stream);
-/* Times candidate launch shapes on the batch (whole tiles, reported with the
- * default `block`, or workgroups of 256/512/1024 lanes x
- * row-major/Morton tile walk x given/heaviest-first job order x LDS stack
+/* Times candidate launch shapes on the batch (whole tiles or workgroups of
+ * 256/512/1024 lanes x row-major/Morton tile walk x given/heaviest-first job order x LDS stack
  * depth: one launch whose stacks fit the deepest tree, or two depth classes
  * split at the depth that halves the batch's work (pixels x depth; failing
  * that, below the deepest trees), each launch's stacks sized to its own
  * deepest tree; `reps` launches each), keeps the fastest for later launches
  * and reports it. */
 typedef struct csg_batch_tuning {
-  int32_t block;
+  int32_t block;  /* workgroup of the per-lane kernel; where whole tiles were faster (csg_batch_whole_tiles)
+                     it is not used, and csg_render_opts.block = 0 gives this choice, another value does not */
   int32_t tile_walk;
   int32_t heaviest_first;
   float ms;  /* mean time of one launch of the batch with this choice */
   int32_t depth_split; /* 0: one launch; d > 0: trees of <= d levels launch apart from deeper ones */
 } csg_batch_tuning;
 csg_status csg_batch_autotune(csg_batch* batch, int32_t reps, void* stream, csg_batch_tuning* chosen);
+/* Sets *whole_tiles to 1 when launches of the batch, as it is now, classify
+ * whole tiles, else to 0. */
+csg_status csg_batch_whole_tiles(const csg_batch* batch, int32_t* whole_tiles);
 csg_status csg_batch_free(csg_batch* batch);
 
 /* Launch geometry of the per-lane kernel for this scene and options on the

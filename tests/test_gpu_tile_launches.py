@@ -93,3 +93,31 @@ def test_large_trees_in_few_tiles(gpu, n, size, others, mode):
     batch.close()
     for sc in (big, wiki, mixed):
         sc.close()
+
+
+def test_the_tuner_says_which_kernel_it_kept(gpu):
+    """What autotune reports gives the same choice again: block 0 where whole tiles were
+    faster, else the reported block (which turns whole tiles off)."""
+    light, phong = C.light(LIGHT), C.phong(*PHONG)
+    specs = [(C.Scene(text), C.camera_look_at(eye, (0, 0, 0), 60), light, phong, size, size,
+              C.alloc_outputs(size, size)) for text, eye, size in S.batch_mix(12, seed=5, resolutions=(128, 256))]
+    jobs = C.make_jobs(specs)
+    for opts, tiles in [({}, True), ({"block": 256}, False), ({"coop": -1}, False)]:
+        batch = C.Batch(jobs, **opts)
+        assert batch.whole_tiles() == tiles, opts
+        batch.close()
+    batch = C.Batch(jobs)
+    t = batch.autotune(reps=2)
+    again = C.Batch(jobs, block=0 if batch.whole_tiles() else t.block, walk=t.tile_walk)
+    assert again.whole_tiles() == batch.whole_tiles()
+    got = []
+    for b in (batch, again):
+        b.launch()
+        torch.cuda.synchronize()
+        got.append([{k: spec[6][k].clone() for k in KEYS} for spec in specs])
+        b.close()
+    for x, y in zip(*got):
+        for key in KEYS:
+            assert torch.equal(x[key].view(torch.uint8), y[key].view(torch.uint8)), key
+    with pytest.raises(C.CsgError):
+        C._check(C.lib().csg_batch_whole_tiles(None, None))
