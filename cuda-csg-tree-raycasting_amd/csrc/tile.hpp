@@ -42,7 +42,9 @@
 //     crossing is depends on when the machine asks.  So the operator above is
 //     sure up to its last crossing at or before t, if it has one, and so on
 //     to the root, whose first crossing is the answer if it is still sure
-//     (most zones lie on the far side of what the ray hits).  A mixed tree of
+//     (most zones lie on the far side of what the ray hits).  An empty list
+//     keeps its zone, as an operand missed there may let the other one appear,
+//     unless an empty operand without a zone empties it.  A mixed tree of
 //     200 at 1023x1023 hands over 70 rays so, 2234 if any such list fails;
 //   * more crossings than the stack holds.
 // A subtree is skipped for lanes whose answer cannot depend on it: an
@@ -593,7 +595,6 @@ __device__ __forceinline__ void TileTrace(const Job& jb, const RayF& r, uint64_t
   float sure = __builtin_inff();
   int sureLevel = 0;
   bool doubts = false;
-  uint64_t cutLists = 0;  // lanes with a list ended at a tie: their zones outlive an empty list
   // frames of the entered operators: lane i holds level i's
   uint32_t fOp = 0, fRight = 0, fMl = 0, fMh = 0, fRl = 0, fRh = 0;
   int d = 0;
@@ -814,6 +815,7 @@ __device__ __forceinline__ void TileTrace(const Job& jb, const RayF& r, uint64_t
       // Each list's zone; where only one has one and that list is a
       // primitive's, the side it is on (CombineSpecial).
       uint32_t own = 0;
+      bool gone = false;  // empty for good: an operand without a zone is, and empties the combination
       if (zones) {
         float l0 = __builtin_inff(), l1 = -__builtin_inff();
         if ((zoneLevels >> d) & 1) {
@@ -833,6 +835,7 @@ __device__ __forceinline__ void TileTrace(const Job& jb, const RayF& r, uint64_t
         own = hasL & !hasR & ((cur & 4u) != 0) ? 1u : 0u;
         own = hasR & !hasL & ((cur & 8u) != 0) ? 2u : own;
         own = on & !cut ? own : 0u;
+        gone = (op != kOpUnion) & (nL == 0 ? !hasL : ((op > kOpDifference) & (nR == 0) & !hasR));
         zlo = fminf(zlo, l0);
         zhi = fmaxf(zhi, l1);
       }
@@ -867,9 +870,7 @@ __device__ __forceinline__ void TileTrace(const Job& jb, const RayF& r, uint64_t
             zlo = ended ? fminf(zlo, __uint_as_float(cutAt)) : zlo;
             zhi = ended ? fmaxf(zhi, end) : zhi;
             bad |= ended & cut;
-            const uint64_t endedLanes = __ballot(ended);
-            zones |= endedLanes != 0;
-            cutLists |= endedLanes;
+            zones |= __ballot(ended) != 0;
             dead |= __ballot(bad);
           }
         }
@@ -885,9 +886,10 @@ __device__ __forceinline__ void TileTrace(const Job& jb, const RayF& r, uint64_t
         const bool drop = !both & (own != 0) & (sp == base + 2) & (t0 >= zlo) & (t0 < zhi);
         sp = drop ? base + 1 : sp;
         zhi = drop ? t0 : zhi;
-        const bool empty = on & (sp == base) & !cut & ((cutLists & me) == 0);
-        zlo = empty ? __builtin_inff() : zlo;
-        zhi = empty ? -__builtin_inff() : zhi;
+        // (a zone no longer than a point is none: it must not widen the next one)
+        gone = (gone & on & !cut) | !(zhi > zlo);
+        zlo = gone ? __builtin_inff() : zlo;
+        zhi = gone ? -__builtin_inff() : zhi;
         // the last crossing a child's doubt leaves sure; none of an empty
         // list that the other child alone has emptied
         bool low = false;
