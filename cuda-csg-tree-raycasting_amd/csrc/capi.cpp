@@ -243,6 +243,7 @@ void LaunchScenes::Add(const csg_scene* s, int64_t tiles, Mode mode) {
   maxOps = std::max(maxOps, ops);
   maxLeaves = std::max(maxLeaves, s->dev.opLeaves);
   inBoxes |= s->dev.conservative != 0;
+  insideOut |= s->flat.insideOut;
   const int64_t flush = s->flat.flushParts, parts = s->flat.nPrims;
   const bool quarter = flush > 0 && kFlushShare * flush >= parts;
   const bool ties = (quarter && ops < kFlushSmallOps) || (tiles >= kTiesTiles && flush * tiles >= kTiesWork * parts);
@@ -264,6 +265,7 @@ void LaunchScenes::Add(const csg_scene* s, int64_t tiles, Mode mode) {
 }
 
 bool LaunchScenes::KeepsLanes(Mode mode) const {
+  if (insideOut) return true;
   double lost = byLanes;
   if (largeWork > 0)
     lost += std::max(kLaneLeastUs,

@@ -37,6 +37,7 @@ inline bool HasTileGroups(const csg_scene* s) { return s->dev.tileOps != s->dev.
 struct LaunchScenes {
   int32_t maxOps, maxLeaves;
   bool inBoxes = false, groups = false;
+  bool insideOut = false;  // boxes that do not hold their subtrees, as whole tiles and groups require
   // what the launch would lose by whole tiles, and what without them (us)
   double byTiles = 0, byLanes = 0;
   double chain = 0;       // of byTiles: the longest walk of a large tree in few tiles, beyond its time per lane

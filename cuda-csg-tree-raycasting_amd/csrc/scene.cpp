@@ -358,7 +358,10 @@ FlatScene Flatten(const CSGTree& tree) {
     f.primB[p] = F4{q.axis[0], q.axis[1], q.axis[2], q.height};
     f.primC[p] = F4{q.r, q.g, q.b, 0.0f};
     if (q.type == kCylinder && !CylinderInBox(q)) f.conservative = false;
+    // a negative size turns its box inside out: the boxes above need not hold it
+    if (s < 0 || (q.type == kCylinder && q.height < 0)) f.insideOut = true;
   }
+  f.conservative &= !f.insideOut;
   if (f.nOps > 0) {
     // Culling boxes for fast mode, each containing what the reference's
     // culling lets a ray see of its subtree, so that they cull the same rays

@@ -114,12 +114,13 @@ struct FlatScene {
   // least kTileGroup members flattened (their chunk and member records are
   // walkOps'); empty where there is none.
   std::vector<F4> tileOps;
+  bool insideOut = false;   // some primitive's size is negative
   int32_t unionGroups = 0;  // Union groups flattened in walkOps
   int32_t flushParts = 0;   // primitives of large Unions that share a face's plane with another member (CountFlush)
   uint32_t rootDesc = 0;
   int32_t nNodes = 0, nOps = 0, nPrims = 0, opDepth = 0;
   int32_t opLeaves = 0;  // operators without an operator child
-  bool conservative = true;  // every primitive lies inside its box (false: a tilted cylinder pokes out)
+  bool conservative = true;  // every primitive lies inside its box (false: a tilted cylinder pokes out, or a size is negative)
 };
 
 constexpr uint32_t kGroupFlag = 0x200u;    // type word bit of a flattened Union group (walkOps)

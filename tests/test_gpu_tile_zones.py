@@ -2,10 +2,12 @@
 box's exit the state machine takes the primitive for missed, also where the
 operator's own list is empty.  Default launches against the per-lane state
 machine (`coop=-1`), bit for bit, and exact mode against the FP32 oracle."""
+import numpy as np
 import pytest
 import torch
 import csgray as C
 import oracle as O
+from csgray import scenes as S
 
 pytestmark = pytest.mark.gpu
 
@@ -92,3 +94,50 @@ def test_a_covered_operand_reappears_beyond_the_box(gpu):
 def test_views_whose_rounding_leaves_the_boxes(gpu, name):
     text, cam, w, h = FAR[name]
     _compare(text, C.camera(*cam, 0.0003490655799396336), w, h)
+
+
+def _inside_out(seed, group):
+    """A tree of 16 parts, or a Union of 30 small Differences, every fourth part of a negative size."""
+    rng = np.random.default_rng(seed)
+
+    def part(i):
+        c, sign, kind = rng.uniform(-0.8, 0.8, 3), (-1.0 if i % 4 == 0 else 1.0), int(rng.integers(0, 3))
+        if kind == 0:
+            return S.sphere(c, "5AC85A", sign * rng.uniform(0.2, 0.6))
+        if kind == 1:
+            return S.cube(c, "C85A5A", sign * rng.uniform(0.3, 0.9))
+        r, h = rng.uniform(0.15, 0.4), rng.uniform(0.4, 1.2)
+        if i % 8 == 4:
+            r, h = r, sign * h
+        else:
+            r = sign * r
+        return S.cylinder(c, "5A5AC8", r, h, rng.uniform(0, 180, 3))
+
+    if group:
+        lines = S.balanced("Union", ["\n".join(["Difference", part(2 * i), part(2 * i + 1)]) for i in range(30)])
+    else:
+        lines = S.random_ops_balanced(rng, [part(i) for i in range(16)])
+    return "\n".join(lines) + "\n"
+
+
+@pytest.mark.parametrize("group", [False, True], ids=["tree", "group"])
+def test_negative_sizes_turn_boxes_inside_out(gpu, group):
+    for seed in range(6):
+        text = _inside_out(seed, group)
+        print(f"[case] seed {seed}", flush=True)
+        for eye in [(2.2, 1.3, 2.9), (0.1, 0.2, 4.0)]:
+            _compare(text, C.camera_look_at(eye, (0, 0.01, 0), 50), 120, 90)
+
+
+def test_negative_sizes_in_a_batch(gpu):
+    light, phong = C.light((0.4, 0.7, 0.6)), C.phong(0.2, 0.7, 0.3, 16.0)
+    cam = C.camera_look_at((2.2, 1.3, 2.9), (0, 0.01, 0), 50)
+    texts = [_inside_out(1, True), S.WIKIPEDIA, _inside_out(2, False), S.cheese(40, seed=40)]
+    specs = [(C.Scene(t), cam, light, phong, 120, 90, C.alloc_outputs(120, 90)) for t in texts]
+    for mode in (C.MODE_FAST, C.MODE_EXACT):
+        refs = [sp[0].render(cam, light, phong, 120, 90, mode=mode, coop=-1) for sp in specs]
+        C.render_batch(C.make_jobs(specs), mode=mode)
+        torch.cuda.synchronize()
+        for spec, ref in zip(specs, refs):
+            for key in ("rgba", "depth", "prim_id", "flags"):
+                assert torch.equal(spec[6][key].view(torch.uint8), ref[key].view(torch.uint8)), key
