@@ -154,13 +154,18 @@ hipError_t DeviceShapeLimits(int* computeUnits, size_t* ldsPerBlock, size_t* lds
 
 // Tile kernel (tile.hpp): entries of a lane's list stack, with Union groups
 // and without.  Fewer leave room for more waves, more hand over fewer rays:
-// the 512-sphere frame takes 215, 210 and 194 us with 24, 26 and 28, but with
-// 28 next to none of its rays go to the cooperative kernel, as callers that
-// watch its counter expect of that frame.
+// the 512-sphere frame takes 215, 210 and 194 us with 24, 26 and 28.  26 is not
+// the fastest there: with 28 default options hand over next to none of that
+// frame's rays, and tests/test_gpu_coop.py expects them to.
 constexpr int32_t kTileSlots = 26, kTilePlainSlots = 16;
-// Exact mode, trees of fewer than kTileLargeOps operators and others.  At
-// 640x360, 24 and 40 slots: unions of 400 541 and 579 us, trees of 200 373 and
-// 378; 512 spheres taken from a cube 973 and 781 us, 1500 4754 and 3975.
+// Exact mode, trees of fewer than kTileLargeOps operators and others, 24 and 40
+// slots, us at 640x360 and 1920x1080: 440 spheres taken from a cube 737 and
+// 683, 1497 and 1753; 500 990 and 791, 1888 and 1957; 800 at 1920x1080 4047 and
+// 3246; unions of 500 spheres 735 and 757, 1841 and 2137, of 1200 at 1920x1080
+// 6644 and 5414; 500 spheres and cylinders taken from a cube 800 and 801, 1612
+// and 1918, 1200 4632 and 4605; mixed trees of 500 40 and 43, 120 and 153, of
+// 1200 at 1920x1080 395 and 496.  (The line suits cut cubes; unions would have it
+// near 1000, mixed trees never.)
 constexpr int32_t kTileLargeOps = 448, kTileExactSmallSlots = 24, kTileExactSlots = 40;
 // A tile's walk of a large tree is one long chain, which few tiles do not
 // hide; the per-lane kernel and a wave a heavy ray are faster for them.  Fast

@@ -304,23 +304,6 @@ __device__ __forceinline__ Hit SphereHit(const RayF& r, const float4& a, uint32_
   return SphereAt(r, a, prim, temp);
 }
 
-// cylinderHit (:202-336).  Both roots go through the same cap logic, as in
-// the reference's duplicated blocks (:238-266, :273-301).
-//
-// Fast mode solves the side's quadratic in the plane across the axis, from
-// the ray's closest approach to the axis (the sphere's closest-approach
-// discriminant carried to that plane).  With e = d x V and g = OC x V (d and
-// OC turned a quarter about V: lengths and dot products as their components
-// across the axis), A = |e|^2, b = e.g, the closest approach lies at
-// tc = -b / A, at distance |g + tc e| from the axis, and the roots are
-// tc -+ sqrt((r^2 - |g + tc e|^2) / A): the reference's (-b -+ sqrt(b^2 - A c)) / A
-// with c = |g|^2 - r^2.  The reference forms c as |OC|^2 - (OC.V)^2 - r^2,
-// which cancels two numbers of the size |OC|^2 and amplifies the rounding of
-// the FP32 axis's length (|OC|^2 (1 - |V|^2)); for thin cylinders seen nearly
-// along their axis that moved depths by 3e-4 relative, while the form here
-// keeps them near 1e-6.  Where the reference's clamp A = 1e-5 applies (rays
-// within 0.18 degrees of the axis) the clamped quadratic is kept:
-// (b^2 - A c) / A = -b tc - c.
 // A ray's two candidate crossings of a cylinder, in the order of the roots:
 // the side's root or, where that lies beyond a cap's plane, the cap (cap 1
 // bottom, 2 top); `skip` where the cap's plane is parallel to the ray.
@@ -332,7 +315,9 @@ struct CylinderRoots {
 };
 
 // False when the ray misses the cylinder's side or passes both caps outside
-// (without a branch).
+// (without a branch; the arithmetic of CylinderHit, expression by expression,
+// as that of RootsOfSphere is SphereRoots's: the two kernels' crossings are
+// compared bit for bit).
 template <bool kFast>
 __device__ __forceinline__ bool RootsOfCylinder(const RayF& r, const float4& a, const float4& bx, CylinderRoots& o) {
   const float vx = bx.x, vy = bx.y, vz = bx.z, height = bx.w, radius = a.w;
@@ -421,6 +406,23 @@ __device__ __forceinline__ Hit CylinderAt(const RayF& r, const CylinderRoots& o,
   return Hit{temp, HitBits(f, kCylinderT, prim)};
 }
 
+// cylinderHit (:202-336).  Both roots go through the same cap logic, as in
+// the reference's duplicated blocks (:238-266, :273-301).
+//
+// Fast mode solves the side's quadratic in the plane across the axis, from
+// the ray's closest approach to the axis (the sphere's closest-approach
+// discriminant carried to that plane).  With e = d x V and g = OC x V (d and
+// OC turned a quarter about V: lengths and dot products as their components
+// across the axis), A = |e|^2, b = e.g, the closest approach lies at
+// tc = -b / A, at distance |g + tc e| from the axis, and the roots are
+// tc -+ sqrt((r^2 - |g + tc e|^2) / A): the reference's (-b -+ sqrt(b^2 - A c)) / A
+// with c = |g|^2 - r^2.  The reference forms c as |OC|^2 - (OC.V)^2 - r^2,
+// which cancels two numbers of the size |OC|^2 and amplifies the rounding of
+// the FP32 axis's length (|OC|^2 (1 - |V|^2)); for thin cylinders seen nearly
+// along their axis that moved depths by 3e-4 relative, while the form here
+// keeps them near 1e-6.  Where the reference's clamp A = 1e-5 applies (rays
+// within 0.18 degrees of the axis) the clamped quadratic is kept:
+// (b^2 - A c) / A = -b tc - c.
 template <bool kFast>
 __device__ __forceinline__ Hit CylinderHit(const RayF& r, const float4& a, const float4& bx, uint32_t prim,
                                            float tmin, Hit h) {

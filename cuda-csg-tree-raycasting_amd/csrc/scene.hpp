@@ -125,7 +125,13 @@ struct FlatScene {
 
 constexpr uint32_t kGroupFlag = 0x200u;    // type word bit of a flattened Union group (walkOps)
 constexpr int32_t kMaxGroupMembers = 1024;  // a group's members are tested 64 a round by one wave
-constexpr int32_t kTileGroup = 24;          // smallest group the tile kernel takes flattened
+// Smallest group the tile kernel takes flattened.  Frames with the group and
+// without it, 640x360 and 1920x1080, us: 16 spheres 20 and 24, 85 and 56, taken
+// from a cube 19 and 27, 57 and 56; 16 mixed parts 42 and 38, 117 and 70; 24
+// spheres 22 and 38, 87 and 71, from a cube 21 and 33, 57 and 60; 24 mixed parts
+// 47 and 49, 138 and 79; 32 spheres 25 and 43, 95 and 87; 32 mixed parts 61 and
+// 88, 149 and 139; 64 mixed parts 71 and 149, 174 and 224.
+constexpr int32_t kTileGroup = 24;
 constexpr int32_t kGroupChunk = 4;          // members under one chunk box
 
 constexpr int32_t kMaxNodes = 65535;       // 16-bit node links

@@ -45,7 +45,7 @@
 //     (most zones lie on the far side of what the ray hits).  An empty list
 //     keeps its zone, as an operand missed there may let the other one appear,
 //     unless an empty operand without a zone empties it.  A mixed tree of
-//     200 at 1023x1023 hands over 70 rays so, 2234 if any such list fails;
+//     200 at 1023x1023 hands over 78 rays so, 2234 if any such list fails;
 //   * more crossings than the stack holds.
 // A subtree is skipped for lanes whose answer cannot depend on it: an
 // Intersection's or a Difference's right child where the left list is empty
@@ -1078,10 +1078,14 @@ __device__ __forceinline__ uint32_t JobOfTile(const Job* jobs, uint32_t n, uint3
 // Walks a tile's rays may take.
 constexpr int kTilePasses = 24;
 // State-machine steps a failed ray takes in its lane before the cooperative
-// kernel gets it.  Most that fail on a tie end within 16, and a launch may
-// then have none to hand over; each step holds the whole wave up for about a
-// microsecond.  1920x1080 at 4 samples of the Wikipedia scene: 0 steps 252,
-// 16 225, 48 227 us; the 512-sphere frame (lists overflow): 236, 243, 259 us.
+// kernel gets it, in launches without groups whose trees have 8 operators or
+// more (others finish it in its lane, or hand it over at once).  Each step
+// holds the whole wave up for about a microsecond, and a launch that hands
+// nothing over saves one ray's chain there.  0, 16, 32 and 64 steps: a mixed tree of
+// 200 at 1023x1023 393, 393, 402 and 427 us; 64 cylinders on a grid at 640x360
+// 137, 145, 155 and 186; 20 cubes on a grid 67, 66, 45 and 45; a plate with 8
+// holes at 1920x1080, exact mode, 75, 67, 68 and 67; 48 random trees in a batch
+// 1426, 1422, 1422 and 1438.
 constexpr int kTileSteps = 16;
 
 // Whether the cooperative kernel has been handed fewer rays than it has waves.
