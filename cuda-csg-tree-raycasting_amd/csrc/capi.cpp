@@ -194,8 +194,8 @@ int32_t DefaultCoopGraceMille(int64_t waves, int64_t tiles, bool batched, bool l
 // ray in a group, while the walk operator by operator follows most ties to
 // their end: no groups for small trees of which a quarter is flush, and for
 // any from kTiesTiles tiles on where flush parts x tiles reach kTiesWork x
-// parts.  On a grid, with the group and without: 24 cubes 320x184 68 and 43 us,
-// 640x360 101 and 46, 1920x1080 447 and 174; 64 cubes 320x184 139 and 157,
+// parts.  On a grid, with the group and without: 24 cubes 640x360 101 and 46 us,
+// 1920x1080 359 and 99; 64 cubes 320x184 139 and 157,
 // 640x360 291 and 172; 200 cubes 480x272 553 and 598, 640x360 776 and 653; 64
 // cylinders (10 of them flush) 640x360 107 and 137, 960x544 143 and 148,
 // 1280x720 201 and 175.

@@ -1081,12 +1081,13 @@ constexpr int kTilePasses = 24;
 // kernel gets it, in launches without groups whose trees have 8 operators or
 // more (others finish it in its lane, or hand it over at once).  Each step
 // holds the whole wave up for about a microsecond, and a launch that hands
-// nothing over saves one ray's chain there.  0, 16, 32 and 64 steps: a mixed tree of
-// 200 at 1023x1023 393, 393, 402 and 427 us; 64 cylinders on a grid at 640x360
-// 137, 145, 155 and 186; 20 cubes on a grid 67, 66, 45 and 45; a plate with 8
+// nothing over saves one ray's chain there, which small trees take with a few
+// more steps.  0, 16, 32 and 64 steps: a union of 20 cubes on a grid at 640x360 67,
+// 66, 45 and 45 us, of 30 223, 218, 214 and 267, of 64 cylinders 137, 145, 155
+// and 186; a mixed tree of 200 at 1023x1023 393, 393, 402 and 427; a plate with 8
 // holes at 1920x1080, exact mode, 75, 67, 68 and 67; 48 random trees in a batch
 // 1426, 1422, 1422 and 1438.
-constexpr int kTileSteps = 16;
+constexpr int kTileSteps = 16, kTileSmallOps = 32, kTileSmallSteps = 32;
 
 // Whether the cooperative kernel has been handed fewer rays than it has waves.
 // Such rays are traced side by side, where a tile's stretches follow one
@@ -1258,7 +1259,8 @@ TileKernel(RenderParams p) {
     // finished here.
     const int depth = max(p.stackSlots, 1), cols = min(64, 64 * (p.tileSlots + 2) / depth);
     bool need = (fail >> lane) & 1u;
-    for (int steps = p.heavyCap != 0 ? (kGroups ? 0 : kTileSteps) : 0x7FFFFFFF;; steps = 0x7FFFFFFF) {
+    const int handSteps = kGroups ? 0 : (p.coopOps < kTileSmallOps ? kTileSmallSteps : kTileSteps);
+    for (int steps = p.heavyCap != 0 ? handSteps : 0x7FFFFFFF;; steps = 0x7FFFFFFF) {
       bool left = steps == 0;
       for (int first = 0; first < 64 && steps != 0; first += cols) {
         if (need & (lane >= first) & (lane < first + cols))

@@ -141,11 +141,13 @@ def _flush_cubes(n, seed, cut=False):
     return "\n".join(S.balanced("Union", leaves)) + "\n"
 
 
-# Unions of flush parts: too few members for a group, a group of few, groups kept up to 3000 tiles
-# (432x432 has 2916, 440x440 3025), and by the per-lane kernel: in fast mode from 48 operators
-# and 6144 tiles on (624x624 has 6084, 632x632 6241), from 400 operators and 3000 tiles in both modes
+# Unions of flush parts: too few members for a group, a group of few, 31 and 32 operators (32 and 16
+# steps in a failed ray's lane), groups kept up to 3000 tiles (432x432 has 2916, 440x440 3025), and by
+# the per-lane kernel: in fast mode from 48 operators and 6144 tiles on (624x624 has 6084, 632x632
+# 6241), from 400 operators and 3000 tiles in both modes
 @pytest.mark.parametrize("mode", [C.MODE_FAST, C.MODE_EXACT], ids=["fast", "exact"])
-@pytest.mark.parametrize("n,cut", [(23, False), (24, False), (24, True), (48, False), (49, False), (200, True), (400, False), (401, False)])
+@pytest.mark.parametrize("n,cut", [(23, False), (24, False), (24, True), (32, False), (33, False), (48, False),
+                                   (49, False), (200, True), (400, False), (401, False)])
 def test_flush_unions_equal_the_state_machine(gpu, n, cut, mode):
     scene = C.Scene(_flush_cubes(n, n, cut))
     specs, refs = [], []

@@ -23,11 +23,12 @@ def _flush_cubes(seed=174):
 
 def test_a_later_launch_of_small_trees_finishes_its_rays(gpu):
     small = C.Scene(_flush_cubes())
-    # nine primitives, out of sight: a launch with this tree has a cooperative kernel, and gives it no rays
-    nine = C.Scene("\n".join(S.balanced("Union", [S.sphere((30 + i, 0, 0), "5AC85A", 0.2) for i in range(9)])) + "\n")
+    # 33 primitives, out of sight: a launch with this tree has a cooperative kernel, which its failed
+    # rays go to after 16 steps, and gives it no rays itself
+    other = C.Scene("\n".join(S.balanced("Union", [S.sphere((30 + i, 0, 0), "5AC85A", 0.2) for i in range(33)])) + "\n")
     cam, light, phong = C.camera_look_at((2.2, 1.3, 2.9), (0, 0, 0), 45), C.light(LIGHT), C.phong(*PHONG)
     ref = small.render(cam, light, phong, 48, 48, coop=-1)
-    far = nine.render(cam, light, phong, 8, 8, coop=-1)
+    far = other.render(cam, light, phong, 8, 8, coop=-1)
     out, rest = C.alloc_outputs(48, 48), [C.alloc_outputs(8, 8) for _ in range(1024)]
 
     def clear():
@@ -38,7 +39,7 @@ def test_a_later_launch_of_small_trees_finishes_its_rays(gpu):
     # in one launch the small tree's rays do go to the cooperative kernel
     clear()
     before = C.coop_rays()
-    C.render_batch(C.make_jobs([(small, cam, light, phong, 48, 48, out), (nine, cam, light, phong, 8, 8, rest[0])]))
+    C.render_batch(C.make_jobs([(small, cam, light, phong, 48, 48, out), (other, cam, light, phong, 8, 8, rest[0])]))
     assert C.coop_rays() > before
     for key in KEYS:
         assert torch.equal(out[key].view(torch.uint8), ref[key].view(torch.uint8)), key
@@ -46,7 +47,7 @@ def test_a_later_launch_of_small_trees_finishes_its_rays(gpu):
     clear()
     before = C.coop_rays()
     print("[case] 1024 + 1 jobs", flush=True)
-    C.render_batch(C.make_jobs([(nine, cam, light, phong, 8, 8, o) for o in rest] +
+    C.render_batch(C.make_jobs([(other, cam, light, phong, 8, 8, o) for o in rest] +
                                [(small, cam, light, phong, 48, 48, out)]))
     assert C.coop_rays() == before
     for key in KEYS:
@@ -55,12 +56,12 @@ def test_a_later_launch_of_small_trees_finishes_its_rays(gpu):
             assert torch.equal(o[key].view(torch.uint8), far[key].view(torch.uint8)), key
     # and the stream's next hand-over finds an empty list
     clear()
-    C.render_batch(C.make_jobs([(small, cam, light, phong, 48, 48, out), (nine, cam, light, phong, 8, 8, rest[0])]))
+    C.render_batch(C.make_jobs([(small, cam, light, phong, 48, 48, out), (other, cam, light, phong, 8, 8, rest[0])]))
     torch.cuda.synchronize()
     for key in KEYS:
         assert torch.equal(out[key].view(torch.uint8), ref[key].view(torch.uint8)), key
     small.close()
-    nine.close()
+    other.close()
 
 
 # A launch keeps the per-lane kernel for large trees with groups in few tiles (64x64: 64 tiles; 1000
