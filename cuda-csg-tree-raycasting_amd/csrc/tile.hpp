@@ -816,7 +816,10 @@ __device__ __forceinline__ void TileTrace(const Job& jb, const RayF& r, uint64_t
       // primitive's, the side it is on (CombineSpecial).
       uint32_t own = 0;
       bool gone = false;  // empty for good: an operand without a zone is, and empties the combination
-      if (zones) {
+      // Whether some lane has a zone or a doubt here (in exact mode, where nearly
+      // every tile has zones, the test costs 8 % of 181 spheres at 1722x1722).
+      bool zoned = zones && (!kFast || doubts || ((zoneLevels >> d) & 1) != 0 || __ballot(zhi > zlo) != 0);
+      if (zoned) {
         float l0 = __builtin_inff(), l1 = -__builtin_inff();
         if ((zoneLevels >> d) & 1) {
           zoneLevels &= ~(uint64_t{1} << d);
@@ -838,6 +841,14 @@ __device__ __forceinline__ void TileTrace(const Job& jb, const RayF& r, uint64_t
         gone = (op != kOpUnion) & (nL == 0 ? !hasL : ((op > kOpDifference) & (nR == 0) & !hasR));
         zlo = fminf(zlo, l0);
         zhi = fmaxf(zhi, l1);
+        // Past the last crossing of an operand without a zone that the solid
+        // lies in, the combination is empty whatever the other one is.
+        if (op != kOpUnion && !cut && __ballot(both & (hasL != hasR)) != 0) {
+          const float lastL = __uint_as_float(EntryTime(list.At(max(mid - 1, 0))));
+          const float lastR = __uint_as_float(EntryTime(list.At(max(sp - 1, 0))));
+          zhi = both & !hasL ? fminf(zhi, lastL) : zhi;
+          zhi = both & (op > kOpDifference) & !hasR ? fminf(zhi, lastR) : zhi;
+        }
       }
       if (__ballot(both) != 0) {
         const uint32_t table = SolidTable(op);
@@ -870,7 +881,8 @@ __device__ __forceinline__ void TileTrace(const Job& jb, const RayF& r, uint64_t
             zlo = ended ? fminf(zlo, __uint_as_float(cutAt)) : zlo;
             zhi = ended ? fmaxf(zhi, end) : zhi;
             bad |= ended & cut;
-            zones |= __ballot(ended) != 0;
+            zoned |= __ballot(ended) != 0;
+            zones |= zoned;
             dead |= __ballot(bad);
           }
         }
@@ -879,13 +891,15 @@ __device__ __forceinline__ void TileTrace(const Job& jb, const RayF& r, uint64_t
       // an Intersection with one list empty, a Difference with the left one
       const bool none = on & !both & ((op > kOpDifference) | ((op == kOpDifference) & (nL == 0)));
       sp = none ? base : sp;
-      if (zones) {
+      if (zoned) {
         // an only list with its own zone: once its Enter is returned in the
         // zone, its Exit is not seen (CombineSpecial)
         const float t0 = __uint_as_float(EntryTime(list.At(base)));
         const bool drop = !both & (own != 0) & (sp == base + 2) & (t0 >= zlo) & (t0 < zhi);
         sp = drop ? base + 1 : sp;
         zhi = drop ? t0 : zhi;
+        // missed, a primitive that the solid lies in leaves it empty too
+        gone |= (sp == base) & ((own == 1 && op != kOpUnion) | (own == 2 && op > kOpDifference));
         // (a zone no longer than a point is none: it must not widen the next one)
         gone = (gone & on & !cut) | !(zhi > zlo);
         zlo = gone ? __builtin_inff() : zlo;
