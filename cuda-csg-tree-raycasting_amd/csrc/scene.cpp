@@ -164,25 +164,23 @@ void AddFaces(const Primitive& q, int32_t member, int32_t prim, std::vector<Face
   }
 }
 
-// How many primitives have a face in one plane with, facing the same way as
+// Marks the primitives with a face in one plane with, facing the same way as
 // and overlapping a face of another member: rays through both cross them at
 // one time (a tie).  Each face is compared with the next kNear of its plane.
-int32_t CountFlush(std::vector<Face>& faces, size_t prims) {
+void MarkFlush(std::vector<Face>& faces, std::vector<uint8_t>* flush) {
   constexpr size_t kNear = 64;
   std::sort(faces.begin(), faces.end(), [](const Face& x, const Face& y) {
     return std::tie(x.side, x.at, x.lo[0]) < std::tie(y.side, y.at, y.lo[0]);
   });
-  std::vector<uint8_t> flush(prims, 0);
   for (size_t i = 0; i < faces.size(); i++) {
     const Face& x = faces[i];
     for (size_t j = i + 1; j < std::min(faces.size(), i + 1 + kNear); j++) {
       const Face& y = faces[j];
       if (y.side != x.side || y.at != x.at || !(y.lo[0] < x.hi[0])) break;
       if (x.member != y.member && x.lo[1] < y.hi[1] && y.lo[1] < x.hi[1])
-        flush[static_cast<size_t>(x.prim)] = flush[static_cast<size_t>(y.prim)] = 1;
+        (*flush)[static_cast<size_t>(x.prim)] = (*flush)[static_cast<size_t>(y.prim)] = 1;
     }
   }
-  return static_cast<int32_t>(std::count(flush.begin(), flush.end(), uint8_t{1}));
 }
 
 }  // namespace
@@ -443,6 +441,7 @@ FlatScene Flatten(const CSGTree& tree) {
     std::vector<int32_t> members, todo;
     std::vector<int32_t> roots;
     std::vector<Face> faces;
+    std::vector<uint8_t> flush(tree.primitives.size(), 0);
     for (int32_t i = 0; i < f.nNodes; i++) {
       const CSGNode& n = tree.nodes[i];
       if (n.primitiveIdx == -1 && n.type == kUnion && (n.parent < 0 || tree.nodes[n.parent].type != kUnion))
@@ -555,10 +554,11 @@ FlatScene Flatten(const CSGTree& tree) {
             }
           }
         }
-        f.flushParts += CountFlush(faces, tree.primitives.size());
+        MarkFlush(faces, &flush);
       }
       f.unionGroups++;
     }
+    f.flushParts = static_cast<int32_t>(std::count(flush.begin(), flush.end(), uint8_t{1}));
   }
   // Groups of few members beside a scene's primitives are not worth the kernel
   // that walks them, which runs half as many waves and goes over a ray whose

@@ -116,7 +116,7 @@ struct FlatScene {
   std::vector<F4> tileOps;
   bool insideOut = false;   // some primitive's size is negative
   int32_t unionGroups = 0;  // Union groups flattened in walkOps
-  int32_t flushParts = 0;   // primitives of large Unions that share a face's plane with another member (CountFlush)
+  int32_t flushParts = 0;   // primitives of large Unions that share a face's plane with another member (MarkFlush)
   uint32_t rootDesc = 0;
   int32_t nNodes = 0, nOps = 0, nPrims = 0, opDepth = 0;
   int32_t opLeaves = 0;  // operators without an operator child
