@@ -299,10 +299,12 @@ csg_status csg_batch_free(csg_batch* batch);
 /* Launch geometry of the per-lane kernel for this scene and options on the
  * current device, for a large frame (no reference counterpart; for tests and
  * tuning).  csg_render_ex uses it when an option shapes it (block, placement,
- * tile order, counters, hand-over, boxes) and for large trees in few tiles;
- * otherwise a workgroup of one wave classifies each 8x8 tile.  A single-scene launch with the scene in LDS takes 1024-lane
- * workgroups when they fit, the scene has at least 256 operators and the frame
- * has an 8x8 tile for every wave of that grid; otherwise 512 lanes. */
+ * tile order, counters, hand-over, boxes), for large trees in few tiles, large
+ * frames of Unions whose parts share many planes and scenes with a negative
+ * size; otherwise a workgroup of one wave classifies each 8x8 tile.  A
+ * single-scene launch with the scene in LDS takes 1024-lane workgroups when
+ * they fit, the scene has at least 256 operators and the frame has an 8x8 tile
+ * for every wave of that grid; otherwise 512 lanes. */
 typedef struct csg_launch_info {
   int32_t block;          /* threads per workgroup */
   int32_t grid;           /* workgroups (persistent: waves pull 8x8 tiles from a queue) */
